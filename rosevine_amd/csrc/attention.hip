@@ -811,13 +811,28 @@ __global__ __launch_bounds__(ST_WAVES * 64) void k_attn_stream(
 //  - p 2^10 likewise, once per stage (p down to 2^-24 has 11 bits or more); a block's p d_v is then
 //    formed in f16 pairs, hi = ph d_v rounded and lo = pl d_v + (ph d_v - hi), whose bracket is exact (a
 //    product of two 11-bit numbers). d_v enters as d_v 2^-E, E the exponent of the largest scale of the
-//    stages so far: exact down to 2^-14 of that largest (and always for scales under 1).
+//    stages so far: exact down to 2^-14 of 2^E, and p d_v to 2^-35 of 2^E.
+// The last is too little for a row whose own scales lie far below 2^E (another block's, a key's that weighs
+// nothing in it or that it does not see). So a wave keeps the smallest scale too, and where one of a workgroup's
+// waves met a 0 or a scale under 2^(E - PF_NEAR), the workgroup walks its stages again with p d_v formed in f32
+// and scaled by its own power of two per row, block and stage: f16 pairs of 2^-24 of a product, or 2^-40 of
+// the row's largest in the stage. (Both walks, 512 tokens in a window of 1024 keys: 101 us, 53 for one in the
+// same run; 500 tokens x 16 heads of 512 on 4,100 keys 583, 247 for one. The pairs of the second walk in every
+// stage of a single one would cost that much always, and a branch per stage 2 to 5% of the first.)
 // Two waves share a SIMD (at most 256 registers: 4 blocks per wave; 8 blocks per wave and one wave per
 // SIMD took 356 us against 274 on hd 512, the waits of one wave having nothing beside them). What bounds
 // it: VALU, about 620 instructions per wave and stage of 4 blocks against 32 MFMAs. Per workgroup and
 // round of stages 3.9 us (500 tokens x 16 heads of 512 on 3,601 to 4,100 keys, 247 us, 257 TFLOP/s of
 // the two products; per-token kernel 1244 us); without the copies 3.4 us.
 constexpr int PF_ROWS = 32, PF_KEYS = 32;
+// With every scale in [2^(E - 11), 2^(E + 1)) a row's block has at least 127 2^(E - 12) from the key of its
+// largest weight (p >= 1/2 there), and the 2^-35 2^E of each other key is 2^-23 of that.
+constexpr int PF_NEAR = 11;
+// the binary16 bits of 2^(E - PF_NEAR), E >= -15 (1, the smallest scale, if that is below it)
+__device__ __forceinline__ uint32_t pf_near_bits(int E) {
+    const int e = E - PF_NEAR;
+    return e >= -14 ? (uint32_t)(e + 15) << 10 : e >= -24 ? 1u << (e + 24) : 1u;
+}
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -895,6 +910,7 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
     constexpr int PK = 10;  // p <= 2^4 and d_v 2^-E < 2: p 2^PK d_v 2^-E < 2^15
     __shared__ __attribute__((aligned(1024))) uint8_t sh[Sh::LDS];
     __shared__ float wm[NT][PF_ROWS], wt[NT][PF_ROWS], wl[NT][PF_ROWS], wmax[WV][PF_ROWS], wus[WV];
+    __shared__ int wapart[WV];
     const int lane = threadIdx.x & 63, lr = lane & 31, hf = lane >> 5;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int team = w / TW, pw = w % TW;  // blocks NBW pw .. NBW pw + NBW - 1 of the team's stages
@@ -957,10 +973,12 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
         }
     };
     const uint32_t akq = lds_addr(kq), avq = lds_addr(vq), aks = lds_addr(ks), avs = lds_addr(vs);
-    if (team < nst) {
+    auto first_copies = [&]() __attribute__((always_inline)) {
+        if (team >= nst) return;
         issue(kg, akq, aks, u0 + team * PF_KEYS);
         issue(vg, avq, avs, u0 + team * PF_KEYS);
-    }
+    };
+    first_copies();
 
     // ---- q: the row's elements 32 b + 16 hf + 8 m .. + 7 of block b are MFMA m's K slots 8 hf ..
     f16x8 qh[NBW][2], ql[NBW][2];
@@ -968,12 +986,13 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
     {
         const float *qr = q + ((size_t)t * n_head + h) * HD + 32 * NBW * pw + 16 * hf;
         float mx = 0.0f;
+        F4u f[4 * NBW];
 #pragma unroll
-        for (int i = 0; i < 4 * NBW; ++i) {
-            const F4u f = *(const F4u *)(qr + 32 * (i / 4) + 4 * (i % 4));
+        for (int i = 0; i < 4 * NBW; ++i) f[i] = *(const F4u *)(qr + 32 * (i / 4) + 4 * (i % 4));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(f.v[e]));
-        }
+        for (int i = 0; i < 4 * NBW; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(f[i].v[e]));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         if constexpr (TW > 1) {  // the row's largest, over the team's waves
             if (hf == 0) wmax[w][lr] = mx;
@@ -983,7 +1002,6 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
         }
         // mx 2^qe in [2^14, 2^15); under 2^-86, where every score is 0 to f32, 2^qe stays at 2^100
         qe = min(100, 14 + 127 - (int)((__float_as_uint(mx) >> 23) & 0xFF));
-        asm volatile("" : : : "memory");  // the row again, block by block, instead of held
 #pragma unroll
         for (int b = 0; b < NBW; ++b) {
 #pragma unroll
@@ -991,11 +1009,11 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
                 uint32_t hi[4], lw[4];
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-                    const F4u f = *(const F4u *)(qr + 32 * b + 8 * m + 4 * u);
+                    const float *v = f[4 * b + 2 * m + u].v;
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
                         f16x2 a, r;
-                        split2_f16(ldexpf(f.v[2 * e], qe), ldexpf(f.v[2 * e + 1], qe), a, r);
+                        split2_f16(ldexpf(v[2 * e], qe), ldexpf(v[2 * e + 1], qe), a, r);
                         hi[2 * u + e] = as_u32(a);
                         lw[2 * u + e] = as_u32(r);
                     }
@@ -1014,13 +1032,10 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
 
     // the row's largest score, the reference m that p is relative to (p = 2^(score L - m)), and the sum
     // of p 2^PK over this lane's keys (its other half: lane ^ 32)
-    float mt = -INFINITY, m = -INFINITY, l = 0.0f;
-    int E = -15;                    // exponent of the largest value scale so far
+    float mt, m, l;
+    int E;          // exponent of the largest value scale so far
+    uint32_t dlow;  // the bits of the smallest of this lane's copies of them
     f32x16 acc[NBW];
-#pragma unroll
-    for (int b = 0; b < NBW; ++b)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[b][i] = 0.0f;
     // LDS offsets of this lane's first key quants and value quants (block 0; block b: ^ 32 b, as a
     // row of 32 NBW bytes is aligned to its size)
     uint32_t kra, vra;
@@ -1034,232 +1049,310 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
         vra = w * Sh::WAVE + Sh::QBYTES + (key * 2 * NBW + (((lane >> 4) & 1) ^ swz(key))) * 16 + 8 * (lane & 1);
     }
 
-    for (int it = 0; it < nit; ++it) {
-        const int s = it * NT + team;
-        const bool live = s < nst, next = s + NT < nst;
-        const int key0 = u0 + s * PF_KEYS;
-        if (!live) {  // a team past its last stage keeps the barriers
-            if constexpr (TW > 1) __builtin_amdgcn_s_barrier();
-            continue;
-        }
-        f32x16 sc;
-        asm volatile("" : "+v"(kra), "+v"(vra));  // the blocks' offsets are formed where they are used
-        // ---- scores: sc[i] = key 16 hf + i of the stage, query row lr
-        loads_left<Sh::NI>();  // the keys are in LDS (the values may be in flight)
-        // a block's key quants and scales are read one block ahead of their use, and its scale
-        // products run under the next block's MFMAs
-        uint4 kw = *(const uint4 *)(sh + kra);
+    // every stage of the team; APART: p d_v in f32 (above)
+    auto walk = [&](auto apart) __attribute__((always_inline)) {
+        constexpr bool APART = decltype(apart)::value;
+        mt = m = -INFINITY;
+        l = 0.0f;
+        E = -15;
+        dlow = 0x7FFFu;
 #pragma unroll
-        for (int i = 0; i < Sh::NS; ++i)
-            *(uint16_t *)(ksp + ((2 * i + hf) * 32 + lr) * 2) = (uint16_t)*(const uint32_t *)(ks + (64 * i + lane) * 4);
-        wave_lds_sync();
-        f32x16 dp;
+        for (int b = 0; b < NBW; ++b)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sc[i] = 0.0f;
-        uint4 dk[2];
-        auto scale = [&](const f32x16 &d, const uint4 (&k)[2]) {
-            const uint32_t dw[8] = {k[0].x, k[0].y, k[0].z, k[0].w, k[1].x, k[1].y, k[1].z, k[1].w};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                sc[2 * e] = fmaf((float)as_f16x2(dw[e]).x, d[2 * e], sc[2 * e]);
-                sc[2 * e + 1] = fmaf((float)as_f16x2(dw[e]).y, d[2 * e + 1], sc[2 * e + 1]);
+            for (int i = 0; i < 16; ++i) acc[b][i] = 0.0f;
+        for (int it = 0; it < nit; ++it) {
+            const int s = it * NT + team;
+            const bool live = s < nst, next = s + NT < nst;
+            const int key0 = u0 + s * PF_KEYS;
+            if (!live) {  // a team past its last stage keeps the barriers
+                if constexpr (TW > 1) __builtin_amdgcn_s_barrier();
+                continue;
             }
-            asm volatile("" : "+v"(sc));  // here, and not where the sums are used
-        };
+            f32x16 sc;
+            asm volatile("" : "+v"(kra), "+v"(vra));  // the blocks' offsets are formed where they are used
+            // ---- scores: sc[i] = key 16 hf + i of the stage, query row lr
+            loads_left<Sh::NI>();  // the keys are in LDS (the values may be in flight)
+            // a block's key quants and scales are read one block ahead of their use, and its scale
+            // products run under the next block's MFMAs
+            uint4 kw = *(const uint4 *)(sh + kra);
 #pragma unroll
-        for (int b = 0; b < NBW; ++b) {
-            const uint4 kn = b + 1 < NBW ? *(const uint4 *)(sh + (kra ^ (32 * (b + 1)))) : kw;
-            const uint4 *dq = (const uint4 *)(ksp + b * 64 + 32 * hf);
-            const uint4 dn[2] = {dq[0], dq[1]};
-            const f16x8 a0 = q8x8_f16(kw.x, kw.y), a1 = q8x8_f16(kw.z, kw.w);
-            f32x16 d;
+            for (int i = 0; i < Sh::NS; ++i)
+                *(uint16_t *)(ksp + ((2 * i + hf) * 32 + lr) * 2) =
+                    (uint16_t)*(const uint32_t *)(ks + (64 * i + lane) * 4);
+            wave_lds_sync();
+            f32x16 dp;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) d[i] = 0.0f;
-            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, ql[b][0], d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, ql[b][1], d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, qh[b][0], d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, qh[b][1], d, 0, 0, 0);
-            if (b > 0) scale(dp, dk);
-            dp = d;
-            kw = kn;
-            dk[0] = dn[0];
-            dk[1] = dn[1];
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        scale(dp, dk);
-        lds_done();
-        if (next) issue(kg, akq, aks, key0 + NT * PF_KEYS);
-        if constexpr (TW > 1) {  // both waves of a team add the same two partial scores
-            float4 *x = (float4 *)(sh + WV * Sh::WAVE) + (it & 1) * WV * 256 + lane;
+            for (int i = 0; i < 16; ++i) sc[i] = 0.0f;
+            uint4 dk[2];
+            auto scale = [&](const f32x16 &d, const uint4 (&k)[2]) {
+                const uint32_t dw[8] = {k[0].x, k[0].y, k[0].z, k[0].w, k[1].x, k[1].y, k[1].z, k[1].w};
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                x[w * 256 + 64 * i] = make_float4(sc[4 * i], sc[4 * i + 1], sc[4 * i + 2], sc[4 * i + 3]);
-            lds_done();
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" : : : "memory");
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {  // (0 + 1) + (2 + 3)
-                const float4 o = x[(w ^ 1) * 256 + 64 * i];
-                sc[4 * i] += o.x;
-                sc[4 * i + 1] += o.y;
-                sc[4 * i + 2] += o.z;
-                sc[4 * i + 3] += o.w;
-                if constexpr (TW == 4) {
-                    const float4 u = x[(w ^ 2) * 256 + 64 * i], v = x[(w ^ 3) * 256 + 64 * i];
-                    sc[4 * i] += u.x + v.x;
-                    sc[4 * i + 1] += u.y + v.y;
-                    sc[4 * i + 2] += u.z + v.z;
-                    sc[4 * i + 3] += u.w + v.w;
+                for (int e = 0; e < 8; ++e) {
+                    sc[2 * e] = fmaf((float)as_f16x2(dw[e]).x, d[2 * e], sc[2 * e]);
+                    sc[2 * e + 1] = fmaf((float)as_f16x2(dw[e]).y, d[2 * e + 1], sc[2 * e + 1]);
                 }
+                asm volatile("" : "+v"(sc));  // here, and not where the sums are used
+            };
+#pragma unroll
+            for (int b = 0; b < NBW; ++b) {
+                const uint4 kn = b + 1 < NBW ? *(const uint4 *)(sh + (kra ^ (32 * (b + 1)))) : kw;
+                const uint4 *dq = (const uint4 *)(ksp + b * 64 + 32 * hf);
+                const uint4 dn[2] = {dq[0], dq[1]};
+                const f16x8 a0 = q8x8_f16(kw.x, kw.y), a1 = q8x8_f16(kw.z, kw.w);
+                f32x16 d;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) d[i] = 0.0f;
+                d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, ql[b][0], d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, ql[b][1], d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, qh[b][0], d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, qh[b][1], d, 0, 0, 0);
+                if (b > 0) scale(dp, dk);
+                dp = d;
+                kw = kn;
+                dk[0] = dn[0];
+                dk[1] = dn[1];
+                __builtin_amdgcn_sched_barrier(0);
             }
-        }
-        // ---- online softmax of the row
-        const bool whole = key0 >= f0 && key0 + PF_KEYS <= f1;  // no key masked for any row
-        uint32_t seen = 0xFFFFu;
-        if (!whole) {
-            seen = 0;
+            scale(dp, dk);
+            lds_done();
+            if (next) issue(kg, akq, aks, key0 + NT * PF_KEYS);
+            if constexpr (TW > 1) {  // both waves of a team add the same two partial scores
+                float4 *x = (float4 *)(sh + WV * Sh::WAVE) + (it & 1) * WV * 256 + lane;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int key = key0 + 16 * hf + i;
-                const bool in = key >= k0 && key < k1;
-                seen |= in ? 1u << i : 0u;
-                sc[i] = in ? sc[i] : -INFINITY;
-            }
-        }
-        float mx = sc[0];
+                for (int i = 0; i < 4; ++i)
+                    x[w * 256 + 64 * i] = make_float4(sc[4 * i], sc[4 * i + 1], sc[4 * i + 2], sc[4 * i + 3]);
+                lds_done();
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" : : : "memory");
 #pragma unroll
-        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, sc[i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        mt = fmaxf(mt, mx);
-
-        // ---- the stage's value scales: their largest, then d_v 2^-E packed as [block][key]
-        if (next) loads_left<Sh::NI>();
-        else loads_left<0>();
-        uint32_t dbits[Sh::NS], dmax = 0, nonfin = 0;
-#pragma unroll
-        for (int i = 0; i < Sh::NS; ++i) {
-            dbits[i] = *(const uint32_t *)(vs + (64 * i + lane) * 4) & 0xFFFFu;
-            const uint32_t mag = dbits[i] & 0x7FFFu;
-            nonfin |= mag >= 0x7C00u ? 1u : 0u;
-            dmax = max(dmax, mag >= 0x7C00u ? 0u : mag);
-        }
-        const int dtop = (int)half32_max((float)dmax);
-        const int En = max(E, (max(__builtin_amdgcn_readlane(dtop, 0), __builtin_amdgcn_readlane(dtop, 32)) >> 10) - 15);
-        // the reference m, a whole number (so that every rescale is exact), moves only when a score
-        // passes it by more than 4 (in log2): p <= 16
-        float corr = ldexpf(1.0f, E - En);
-        E = En;
-        const float ml = mt * L;
-        if (__builtin_amdgcn_ballot_w64(ml - m > 4.0f || m == -INFINITY)) {
-            const float up = ceilf(ml);
-            const float f = up == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - up);  // 0 while m = -inf
-            m = up;
-            corr *= f;
-            l *= f;
-        }
-#pragma unroll
-        for (int i = 0; i < Sh::NS; ++i) {  // infinite and NaN scales are added below
-            const bool fin = (dbits[i] & 0x7C00u) != 0x7C00u;
-            *(_Float16 *)(vsp + ((2 * i + hf) * 32 + lr) * 2) =
-                (_Float16)(fin ? ldexpf(h2f((uint16_t)dbits[i]), -E) : 0.0f);
-        }
-        if (__builtin_amdgcn_ballot_w64(corr != 1.0f)) {
-#pragma unroll
-            for (int b = 0; b < NBW; ++b)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) acc[b][i] *= corr;
-        }
-        // p 2^PK, from a reference PK lower
-        const float mr = (float)PK - (m == -INFINITY ? 0.0f : m);
-        float ps = 0.0f;
-        f16x2 ph[8], pl[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            sc[2 * i] = __builtin_amdgcn_exp2f(fmaf(sc[2 * i], L, mr));
-            sc[2 * i + 1] = __builtin_amdgcn_exp2f(fmaf(sc[2 * i + 1], L, mr));
-            ps += sc[2 * i] + sc[2 * i + 1];
-            split2_f16(sc[2 * i], sc[2 * i + 1], ph[i], pl[i]);
-        }
-        l += ps;
-        wave_lds_sync();
-        if (__builtin_amdgcn_ballot_w64(nonfin)) {
-            uint32_t sk = 0, pk = 0;  // this row's keys by stage position: seen, and of weight above 0
-#pragma unroll
-            for (int i = 0; i < 16; ++i) pk |= sc[i] > 0.0f ? 1u << i : 0u;
-            sk = seen << (16 * hf);
-            pk <<= 16 * hf;
-            sk |= (uint32_t)__shfl_xor((int)sk, 32);
-            pk |= (uint32_t)__shfl_xor((int)pk, 32);
-#pragma unroll
-            for (int b = 0; b < NBW; ++b)
-#pragma unroll 1
-                for (int key = 0; key < PF_KEYS; ++key) {
-                    const uint32_t db = *(const uint32_t *)(vs + (32 * b + key) * 4) & 0xFFFFu;
-                    if ((db & 0x7C00u) != 0x7C00u) continue;
-                    const float d = sk >> key & 1 ? (pk >> key & 1 ? h2f((uint16_t)db) : NAN) : 0.0f;
-#pragma unroll
-                    for (int i4 = 0; i4 < 4; ++i4) {  // quants of dimensions 8 i4 + 4 hf .. + 3
-                        const int piece = (2 * b + (i4 >> 1)) ^ swz(key);
-                        const uint32_t u =
-                            *(const uint32_t *)(vq + (key * 2 * NBW + piece) * 16 + 8 * (i4 & 1) + 4 * hf);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const float add = d * q8_at(u, e);
-                            acc[b][4 * i4 + e] += sk >> key & 1 ? add : 0.0f;
-                        }
+                for (int i = 0; i < 4; ++i) {  // (0 + 1) + (2 + 3)
+                    const float4 o = x[(w ^ 1) * 256 + 64 * i];
+                    sc[4 * i] += o.x;
+                    sc[4 * i + 1] += o.y;
+                    sc[4 * i + 2] += o.z;
+                    sc[4 * i + 3] += o.w;
+                    if constexpr (TW == 4) {
+                        const float4 u = x[(w ^ 2) * 256 + 64 * i], v = x[(w ^ 3) * 256 + 64 * i];
+                        sc[4 * i] += u.x + v.x;
+                        sc[4 * i + 1] += u.y + v.y;
+                        sc[4 * i + 2] += u.z + v.z;
+                        sc[4 * i + 3] += u.w + v.w;
                     }
                 }
-        }
-
-        // ---- values: acc[b][i] = dimension 32 b + 8 (i / 4) + 4 hf + i % 4, query row lr
-        v2i_t vt[2];
-        uint4 dv[2];
-        auto read_values = [&](int b, v2i_t (&vv)[2], uint4 (&dd)[2]) {
-            const uint8_t *src = sh + (vra ^ (32 * b));
-            vv[0] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t *)src);
-            vv[1] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t *)(src + 256 * NBW));  // 8 keys on
-            const uint4 *dq = (const uint4 *)(vsp + b * 64 + 32 * hf);
-            dd[0] = dq[0];
-            dd[1] = dq[1];
-        };
-        read_values(0, vt, dv);
+            }
+            // ---- online softmax of the row
+            const bool whole = key0 >= f0 && key0 + PF_KEYS <= f1;  // no key masked for any row
+            uint32_t seen = 0xFFFFu;
+            if (!whole) {
+                seen = 0;
 #pragma unroll
-        for (int b = 0; b < NBW; ++b) {
-            v2i_t vn[2] = {vt[0], vt[1]};
-            uint4 dn[2] = {dv[0], dv[1]};
-            if (b + 1 < NBW) read_values(b + 1, vn, dn);
-            f16x8 a[2];
-            uint32_t bh[2][4], bl[2][4];
-#pragma unroll
-            for (int mm = 0; mm < 2; ++mm) {
-                a[mm] = q8x8_f16((uint32_t)vt[mm].x, (uint32_t)vt[mm].y);
-                const uint32_t dw[4] = {dv[mm].x, dv[mm].y, dv[mm].z, dv[mm].w};
-#pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    const f16x2 d2 = as_f16x2(dw[x]), hi = ph[4 * mm + x] * d2;
-                    bh[mm][x] = as_u32(hi);
-                    bl[mm][x] = as_u32(__builtin_elementwise_fma(
-                        pl[4 * mm + x], d2, __builtin_elementwise_fma(ph[4 * mm + x], d2, -hi)));
+                for (int i = 0; i < 16; ++i) {
+                    const int key = key0 + 16 * hf + i;
+                    const bool in = key >= k0 && key < k1;
+                    seen |= in ? 1u << i : 0u;
+                    sc[i] = in ? sc[i] : -INFINITY;
                 }
             }
-            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], as_f16x8(bl[0]), acc[b], 0, 0, 0);
-            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], as_f16x8(bl[1]), acc[b], 0, 0, 0);
-            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], as_f16x8(bh[0]), acc[b], 0, 0, 0);
-            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], as_f16x8(bh[1]), acc[b], 0, 0, 0);
-            vt[0] = vn[0];
-            vt[1] = vn[1];
-            dv[0] = dn[0];
-            dv[1] = dn[1];
-            if (b % 2) __builtin_amdgcn_sched_barrier(0);
+            float mx = sc[0];
+#pragma unroll
+            for (int i = 1; i < 16; ++i) mx = fmaxf(mx, sc[i]);
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            mt = fmaxf(mt, mx);
+
+            // ---- the stage's value scales: their largest, then d_v 2^-E packed as [block][key]
+            if (next) loads_left<Sh::NI>();
+            else loads_left<0>();
+            uint32_t dbits[Sh::NS], dmax = 0, nonfin = 0;
+#pragma unroll
+            for (int i = 0; i < Sh::NS; ++i) {
+                dbits[i] = *(const uint32_t *)(vs + (64 * i + lane) * 4) & 0xFFFFu;
+                const uint32_t mag = dbits[i] & 0x7FFFu;
+                nonfin |= mag >= 0x7C00u ? 1u : 0u;
+                dmax = max(dmax, mag >= 0x7C00u ? 0u : mag);
+                if constexpr (!APART) dlow = min(dlow, mag);
+            }
+            const int dtop = (int)half32_max((float)dmax);
+            const int En =
+                max(E, (max(__builtin_amdgcn_readlane(dtop, 0), __builtin_amdgcn_readlane(dtop, 32)) >> 10) - 15);
+            // the reference m, a whole number (so that every rescale is exact), moves only when a score
+            // passes it by more than 4 (in log2): p <= 16
+            float corr = ldexpf(1.0f, E - En);
+            E = En;
+            const float ml = mt * L;
+            if (__builtin_amdgcn_ballot_w64(ml - m > 4.0f || m == -INFINITY)) {
+                const float up = ceilf(ml);
+                const float f = up == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - up);  // 0 while m = -inf
+                m = up;
+                corr *= f;
+                l *= f;
+            }
+#pragma unroll
+            for (int i = 0; i < Sh::NS; ++i) {  // infinite and NaN scales are added below
+                const bool fin = (dbits[i] & 0x7C00u) != 0x7C00u;
+                *(_Float16 *)(vsp + ((2 * i + hf) * 32 + lr) * 2) =
+                    (_Float16)(fin ? ldexpf(h2f((uint16_t)dbits[i]), APART ? 0 : -E) : 0.0f);
+            }
+            if (__builtin_amdgcn_ballot_w64(corr != 1.0f)) {
+#pragma unroll
+                for (int b = 0; b < NBW; ++b)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[b][i] *= corr;
+            }
+            // p 2^PK, from a reference PK lower
+            const float mr = (float)PK - (m == -INFINITY ? 0.0f : m);
+            float ps = 0.0f;
+            f16x2 ph[8], pl[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                sc[2 * i] = __builtin_amdgcn_exp2f(fmaf(sc[2 * i], L, mr));
+                sc[2 * i + 1] = __builtin_amdgcn_exp2f(fmaf(sc[2 * i + 1], L, mr));
+                ps += sc[2 * i] + sc[2 * i + 1];
+                split2_f16(sc[2 * i], sc[2 * i + 1], ph[i], pl[i]);
+            }
+            l += ps;
+            wave_lds_sync();
+            if (__builtin_amdgcn_ballot_w64(nonfin)) {
+                uint32_t sk = 0, pk = 0;  // this row's keys by stage position: seen, and of weight above 0
+#pragma unroll
+                for (int i = 0; i < 16; ++i) pk |= sc[i] > 0.0f ? 1u << i : 0u;
+                sk = seen << (16 * hf);
+                pk <<= 16 * hf;
+                sk |= (uint32_t)__shfl_xor((int)sk, 32);
+                pk |= (uint32_t)__shfl_xor((int)pk, 32);
+#pragma unroll
+                for (int b = 0; b < NBW; ++b)
+#pragma unroll 1
+                    for (int key = 0; key < PF_KEYS; ++key) {
+                        const uint32_t db = *(const uint32_t *)(vs + (32 * b + key) * 4) & 0xFFFFu;
+                        if ((db & 0x7C00u) != 0x7C00u) continue;
+                        const float d = sk >> key & 1 ? (pk >> key & 1 ? h2f((uint16_t)db) : NAN) : 0.0f;
+#pragma unroll
+                        for (int i4 = 0; i4 < 4; ++i4) {  // quants of dimensions 8 i4 + 4 hf .. + 3
+                            const int piece = (2 * b + (i4 >> 1)) ^ swz(key);
+                            const uint32_t u =
+                                *(const uint32_t *)(vq + (key * 2 * NBW + piece) * 16 + 8 * (i4 & 1) + 4 * hf);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const float add = d * q8_at(u, e);
+                                acc[b][4 * i4 + e] += sk >> key & 1 ? add : 0.0f;
+                            }
+                        }
+                    }
+            }
+
+            // ---- values: acc[b][i] = dimension 32 b + 8 (i / 4) + 4 hf + i % 4, query row lr
+            v2i_t vt[2];
+            uint4 dv[2];
+            auto read_quants = [&](int b, v2i_t (&vv)[2]) {
+                const uint8_t *src = sh + (vra ^ (32 * b));
+                vv[0] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t *)src);
+                vv[1] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t *)(src + 256 * NBW));  // 8 keys on
+            };
+            if constexpr (APART) {
+#pragma unroll
+                for (int b = 0; b < NBW; ++b) {
+                    // the products of keys 4 n .. 4 n + 3 of the lane's 16, formed twice instead of held
+                    float wv[4];
+                    auto products = [&](int n) {
+                        asm volatile("" : : : "memory");
+                        const uint2 r = *(const uint2 *)(vsp + b * 64 + 32 * hf + 8 * n);
+                        const f16x2 d0 = as_f16x2(r.x), d1 = as_f16x2(r.y);
+                        wv[0] = sc[4 * n] * (float)d0.x;
+                        wv[1] = sc[4 * n + 1] * (float)d0.y;
+                        wv[2] = sc[4 * n + 2] * (float)d1.x;
+                        wv[3] = sc[4 * n + 3] * (float)d1.y;
+                    };
+                    float top = 0.0f, sum = 0.0f;
+#pragma unroll
+                    for (int n = 0; n < 4; ++n) {
+                        products(n);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) top = fmaxf(top, fabsf(wv[e]));
+                    }
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) sum = fmaxf(sum, fabsf(acc[b][i]));
+                    // times 2^up the products lie under 2^15, the sums so far under 2^100, in both of the row's lanes
+                    int up = min(141 - (int)((__float_as_uint(top) >> 23) & 0xFF),
+                                 226 - E - (int)((__float_as_uint(sum) >> 23) & 0xFF));
+                    up = min(up, __shfl_xor(up, 32));
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[b][i] = ldexpf(acc[b][i], up + E);
+                    read_quants(b, vt);
+#pragma unroll
+                    for (int mm = 0; mm < 2; ++mm) {
+                        uint32_t bh[4], bl[4];
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            if (x % 2 == 0) products(2 * mm + x / 2);
+                            f16x2 hi, lw;
+                            split2_f16(ldexpf(wv[2 * (x % 2)], up), ldexpf(wv[2 * (x % 2) + 1], up), hi, lw);
+                            bh[x] = as_u32(hi);
+                            bl[x] = as_u32(lw);
+                        }
+                        const f16x8 a = q8x8_f16((uint32_t)vt[mm].x, (uint32_t)vt[mm].y);
+                        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, as_f16x8(bl), acc[b], 0, 0, 0);
+                        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, as_f16x8(bh), acc[b], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[b][i] = ldexpf(acc[b][i], -up - E);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+                auto read_values = [&](int b, v2i_t (&vv)[2], uint4 (&dd)[2]) {
+                    read_quants(b, vv);
+                    const uint4 *dq = (const uint4 *)(vsp + b * 64 + 32 * hf);
+                    dd[0] = dq[0];
+                    dd[1] = dq[1];
+                };
+                read_values(0, vt, dv);
+#pragma unroll
+                for (int b = 0; b < NBW; ++b) {
+                    v2i_t vn[2] = {vt[0], vt[1]};
+                    uint4 dn[2] = {dv[0], dv[1]};
+                    if (b + 1 < NBW) read_values(b + 1, vn, dn);
+                    f16x8 a[2];
+                    uint32_t bh[2][4], bl[2][4];
+#pragma unroll
+                    for (int mm = 0; mm < 2; ++mm) {
+                        a[mm] = q8x8_f16((uint32_t)vt[mm].x, (uint32_t)vt[mm].y);
+                        const uint32_t dw[4] = {dv[mm].x, dv[mm].y, dv[mm].z, dv[mm].w};
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            const f16x2 d2 = as_f16x2(dw[x]), hi = ph[4 * mm + x] * d2;
+                            bh[mm][x] = as_u32(hi);
+                            bl[mm][x] = as_u32(__builtin_elementwise_fma(
+                                pl[4 * mm + x], d2, __builtin_elementwise_fma(ph[4 * mm + x], d2, -hi)));
+                        }
+                    }
+                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], as_f16x8(bl[0]), acc[b], 0, 0, 0);
+                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], as_f16x8(bl[1]), acc[b], 0, 0, 0);
+                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], as_f16x8(bh[0]), acc[b], 0, 0, 0);
+                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], as_f16x8(bh[1]), acc[b], 0, 0, 0);
+                    vt[0] = vn[0];
+                    vt[1] = vn[1];
+                    dv[0] = dn[0];
+                    dv[1] = dn[1];
+                    if (b % 2) __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            lds_done();
+            if (next) issue(vg, avq, avs, key0 + NT * PF_KEYS);
         }
-        lds_done();
-        if (next) issue(vg, avq, avs, key0 + NT * PF_KEYS);
+    };
+    walk(std::false_type{});
+    const bool apart = __builtin_amdgcn_ballot_w64(dlow < pf_near_bits(E)) != 0;
+    if (lane == 0) wapart[w] = apart;
+    __syncthreads();  // every wave is done with its stages
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(wapart[lane % WV] != 0) != 0, 0)) {
+        first_copies();
+        walk(std::true_type{});
+        __syncthreads();
     }
 
     // ---- the teams' results meet in LDS: M = max of their maxima, the sums weighted by e^(m - M);
     // wave (team, pw) finishes a share of its blocks' registers
     l += __shfl_xor(l, 32);
-    __syncthreads();  // every wave is done with its stages
     float *mrg = (float *)sh;  // [wave][block, register][lane]
 #pragma unroll
     for (int b = 0; b < NBW; ++b)
