@@ -813,8 +813,10 @@ __global__ __launch_bounds__(ST_WAVES * 64) void k_attn_stream(
 //    product of two 11-bit numbers). d_v enters as d_v 2^-E, E the exponent of the largest scale of the
 //    stages so far: exact down to 2^-14 of 2^E, and p d_v to 2^-35 of 2^E.
 // The last is too little for a row whose own scales lie far below 2^E (another block's, a key's that weighs
-// nothing in it or that it does not see). So a wave keeps the smallest scale too, and where one of a workgroup's
-// waves met a 0 or a scale under 2^(E - PF_NEAR), the workgroup walks its stages again with p d_v formed in f32
+// nothing in it or that it does not see), as 2^-40 of a row's q is for a block of it that meets large key scales.
+// So a wave keeps the smallest scale too, and where one of a workgroup's waves met a 0 or a scale under
+// 2^(E - PF_NEAR), or a block of q under 2^-PF_Q of its row, the workgroup walks its stages again: such a
+// block of q has a power of two of its own (2^-28 of the block's largest throughout), and p d_v is formed in f32
 // and scaled by its own power of two per row, block and stage: f16 pairs of 2^-24 of a product, or 2^-40 of
 // the row's largest in the stage. (Both walks, 512 tokens in a window of 1024 keys: 101 us, 53 for one in the
 // same run; 500 tokens x 16 heads of 512 on 4,100 keys 583, 247 for one. The pairs of the second walk in every
@@ -827,7 +829,7 @@ __global__ __launch_bounds__(ST_WAVES * 64) void k_attn_stream(
 constexpr int PF_ROWS = 32, PF_KEYS = 32;
 // With every scale in [2^(E - 11), 2^(E + 1)) a row's block has at least 127 2^(E - 12) from the key of its
 // largest weight (p >= 1/2 there), and the 2^-35 2^E of each other key is 2^-23 of that.
-constexpr int PF_NEAR = 11;
+constexpr int PF_NEAR = 11, PF_Q = 12;
 // the binary16 bits of 2^(E - PF_NEAR), E >= -15 (1, the smallest scale, if that is below it)
 __device__ __forceinline__ uint32_t pf_near_bits(int E) {
     const int e = E - PF_NEAR;
@@ -910,7 +912,7 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
     constexpr int PK = 10;  // p <= 2^4 and d_v 2^-E < 2: p 2^PK d_v 2^-E < 2^15
     __shared__ __attribute__((aligned(1024))) uint8_t sh[Sh::LDS];
     __shared__ float wm[NT][PF_ROWS], wt[NT][PF_ROWS], wl[NT][PF_ROWS], wmax[WV][PF_ROWS], wus[WV];
-    __shared__ int wapart[WV];
+    __shared__ int wapart[WV], qdiff[WV][NBW][PF_ROWS];
     const int lane = threadIdx.x & 63, lr = lane & 31, hf = lane >> 5;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int team = w / TW, pw = w % TW;  // blocks NBW pw .. NBW pw + NBW - 1 of the team's stages
@@ -982,18 +984,24 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
 
     // ---- q: the row's elements 32 b + 16 hf + 8 m .. + 7 of block b are MFMA m's K slots 8 hf ..
     f16x8 qh[NBW][2], ql[NBW][2];
-    int qe;  // q is scaled by 2^qe
+    int qe;       // q is scaled by 2^qe,
+    bool qapart;  // block b of some rows by 2^(qe - qdiff[w][b][row])
     {
         const float *qr = q + ((size_t)t * n_head + h) * HD + 32 * NBW * pw + 16 * hf;
-        float mx = 0.0f;
+        float mx = 0.0f, mb[NBW];
         F4u f[4 * NBW];
 #pragma unroll
         for (int i = 0; i < 4 * NBW; ++i) f[i] = *(const F4u *)(qr + 32 * (i / 4) + 4 * (i % 4));
 #pragma unroll
-        for (int i = 0; i < 4 * NBW; ++i)
+        for (int b = 0; b < NBW; ++b) {
+            mb[b] = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(f[i].v[e]));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+            for (int i = 4 * b; i < 4 * b + 4; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) mb[b] = fmaxf(mb[b], fabsf(f[i].v[e]));
+            mb[b] = fmaxf(mb[b], __shfl_xor(mb[b], 32));
+            mx = fmaxf(mx, mb[b]);
+        }
         if constexpr (TW > 1) {  // the row's largest, over the team's waves
             if (hf == 0) wmax[w][lr] = mx;
             __syncthreads();
@@ -1001,9 +1009,19 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
             for (int i = 0; i < TW; ++i) mx = fmaxf(mx, wmax[team * TW + i][lr]);
         }
         // mx 2^qe in [2^14, 2^15); under 2^-86, where every score is 0 to f32, 2^qe stays at 2^100
-        qe = min(100, 14 + 127 - (int)((__float_as_uint(mx) >> 23) & 0xFF));
+        auto up = [](float top) { return min(100, 14 + 127 - (int)((__float_as_uint(top) >> 23) & 0xFF)); };
+        qe = up(mx);
+        bool low = false;
+#pragma unroll
+        for (int b = 0; b < NBW; ++b) low |= mb[b] > 0.0f && mb[b] < ldexpf(mx, -PF_Q);
+        qapart = __builtin_amdgcn_ballot_w64(low) != 0;
 #pragma unroll
         for (int b = 0; b < NBW; ++b) {
+            int qb = qe;
+            if (qapart) {
+                if (mb[b] > 0.0f && mb[b] < ldexpf(mx, -PF_Q)) qb = up(mb[b]);
+                qdiff[w][b][lr] = qe - qb;
+            }
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
                 uint32_t hi[4], lw[4];
@@ -1013,7 +1031,7 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
                         f16x2 a, r;
-                        split2_f16(ldexpf(v[2 * e], qe), ldexpf(v[2 * e + 1], qe), a, r);
+                        split2_f16(ldexpf(v[2 * e], qb), ldexpf(v[2 * e + 1], qb), a, r);
                         hi[2 * u + e] = as_u32(a);
                         lw[2 * u + e] = as_u32(r);
                     }
@@ -1084,7 +1102,12 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
 #pragma unroll
             for (int i = 0; i < 16; ++i) sc[i] = 0.0f;
             uint4 dk[2];
-            auto scale = [&](const f32x16 &d, const uint4 (&k)[2]) {
+            auto scale = [&](f32x16 &d, const uint4 (&k)[2], int b) {
+                if (APART && qapart) {
+                    const int by = qdiff[w][b][lr];
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) d[i] = ldexpf(d[i], by);
+                }
                 const uint32_t dw[8] = {k[0].x, k[0].y, k[0].z, k[0].w, k[1].x, k[1].y, k[1].z, k[1].w};
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
@@ -1106,14 +1129,14 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
                 d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, ql[b][1], d, 0, 0, 0);
                 d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, qh[b][0], d, 0, 0, 0);
                 d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, qh[b][1], d, 0, 0, 0);
-                if (b > 0) scale(dp, dk);
+                if (b > 0) scale(dp, dk, b - 1);
                 dp = d;
                 kw = kn;
                 dk[0] = dn[0];
                 dk[1] = dn[1];
                 __builtin_amdgcn_sched_barrier(0);
             }
-            scale(dp, dk);
+            scale(dp, dk, NBW - 1);
             lds_done();
             if (next) issue(kg, akq, aks, key0 + NT * PF_KEYS);
             if constexpr (TW > 1) {  // both waves of a team add the same two partial scores
@@ -1341,7 +1364,7 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
         }
     };
     walk(std::false_type{});
-    const bool apart = __builtin_amdgcn_ballot_w64(dlow < pf_near_bits(E)) != 0;
+    const bool apart = qapart || __builtin_amdgcn_ballot_w64(dlow < pf_near_bits(E)) != 0;
     if (lane == 0) wapart[w] = apart;
     __syncthreads();  // every wave is done with its stages
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(wapart[lane % WV] != 0) != 0, 0)) {
