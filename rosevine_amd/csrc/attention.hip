@@ -927,7 +927,7 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
     const int pos = p0 + t;
     const int lo = window > 0 ? max(0, pos + 1 - window) : 0;
     const int per = (pos - lo + 1 + n_chunks - 1) / n_chunks;
-    const int k0 = lo + c * per, k1 = min(pos + 1, k0 + per);
+    const int k0 = lo + c * per, k1 = k0 + min(per, pos + 1 - k0);
     const int u0 = __builtin_amdgcn_readlane(k0, 0), u1 = __builtin_amdgcn_readlane(k1, 31);  // any row's
     const int f0 = __builtin_amdgcn_readlane(k0, 31), f1 = __builtin_amdgcn_readlane(k1, 0);  // every row's
     const int nst = u1 > u0 ? (u1 - u0 + PF_KEYS - 1) / PF_KEYS : 0, nit = (nst + NT - 1) / NT;
@@ -956,7 +956,8 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
     for (int i = 0; i < Sh::NS; ++i) soff[i] = (uint32_t)lr * (uint32_t)slot_bytes + Q8_BLOCK * (2 * i + hf);
     auto issue = [&](const uint8_t *base, uint32_t dq, uint32_t ds, int key0) {
         const int s0 = key0 % cap;
-        if (key0 + PF_KEYS <= u1 && s0 + PF_KEYS <= cap) {  // a whole stage without a wrap
+        const int last = u1 - 1 - key0;  // (positions reach 2^31 - 1: here and below key0 + 32 may not fit an int)
+        if (last >= PF_KEYS - 1 && s0 + PF_KEYS <= cap) {  // a whole stage without a wrap
             const uint8_t *b = base + (size_t)s0 * slot_bytes;
 #pragma unroll
             for (int i = 0; i < Sh::NQ; ++i) lds_copy16_at(b, qoff[i], dq + i * 1024);
@@ -965,10 +966,10 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
         } else {  // keys past the last repeat it
 #pragma unroll 1
             for (int i = 0; i < Sh::NQ; ++i) {
-                const int sl = (int)((uint32_t)min(key0 + copy_key(i), u1 - 1) % (uint32_t)cap);
+                const int sl = (int)((uint32_t)(key0 + min(copy_key(i), last)) % (uint32_t)cap);
                 lds_copy16(base + (size_t)sl * slot_bytes + copy_off(i), dq + i * 1024);
             }
-            const int sl = (int)((uint32_t)min(key0 + lr, u1 - 1) % (uint32_t)cap);
+            const int sl = (int)((uint32_t)(key0 + min(lr, last)) % (uint32_t)cap);
 #pragma unroll 1
             for (int i = 0; i < Sh::NS; ++i)
                 lds_copy4(base + (size_t)sl * slot_bytes + Q8_BLOCK * (2 * i + hf), ds + i * 256);
@@ -1164,14 +1165,14 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
                 }
             }
             // ---- online softmax of the row
-            const bool whole = key0 >= f0 && key0 + PF_KEYS <= f1;  // no key masked for any row
+            const bool whole = key0 >= f0 && f1 - key0 >= PF_KEYS;  // no key masked for any row
             uint32_t seen = 0xFFFFu;
             if (!whole) {
                 seen = 0;
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    const int key = key0 + 16 * hf + i;
-                    const bool in = key >= k0 && key < k1;
+                    const uint32_t key = (uint32_t)key0 + 16 * hf + i;
+                    const bool in = key >= (uint32_t)k0 && key < (uint32_t)k1;
                     seen |= in ? 1u << i : 0u;
                     sc[i] = in ? sc[i] : -INFINITY;
                 }
