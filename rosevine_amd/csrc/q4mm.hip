@@ -7,11 +7,12 @@
 // tokens of the call nor on the launch shape (hip_ops.rs:73-78):
 //  - a row's nb blocks fall into four parts of q4_part(nb) blocks;
 //  - the token's activations of a block are scaled by 2^(141 - E), E the largest biased exponent of the
-//    part's blocks up to this one (so that the largest lies under 2^15), and split into two f16, each
-//    rounded: 2^-24 of the element, or 2^-40 of that largest for smaller ones;
+//    part's blocks up to this one (so that the largest lies under 2^15), or the block's own where that is
+//    more than Q4_NEAR lower (q4_exponent), and split into two f16, each rounded: 2^-24 of the element, or
+//    2^-24 of the block's largest for smaller ones;
 //  - n - 8 is exact in f16, so v_mfma_f32_16x16x32_f16 sums exact products over one block: the low
 //    halves first, the high halves onto them;
-//  - acc = fma(d, sum, acc) in block order from 0; where E grows, acc is first scaled to the new one;
+//  - acc = fma(d, sum, acc) in block order from 0; where E changes, acc is first scaled to the new one;
 //  - the parts' sums, scaled back, add as (P0 + P1) + (P2 + P3).
 // A non-finite activation makes the token's results NaN.
 //
@@ -111,6 +112,15 @@ __device__ __forceinline__ void rows_gather(uint32_t s, uint32_t (&v)[4]) {
 
 __device__ __forceinline__ int exp_field(float m) { return (int)((__float_as_uint(m) >> 23) & 0xFF); }
 
+// The exponent that a block's activations are scaled by: own is the block's largest (0: zeros, whose scale
+// does not matter, and subnormal values), top the part's largest up to it. A block far below top would keep
+// few of its bits under top's scale, which a row needs whose weights of the large blocks are as much smaller
+// than this one's, or zeros. 60 below top it stays: the sums so far must not pass the largest float.
+constexpr int Q4_NEAR = 16, Q4_FAR = 60;
+__device__ __forceinline__ int q4_exponent(int own, int top) {
+    return own == 0 || own >= top - Q4_NEAR ? top : max(own, top - Q4_FAR);
+}
+
 // rows of an even block count on a 4-byte aligned matrix: every pair of blocks starts on a dword
 __host__ __device__ __forceinline__ bool q4_rows_aligned(const uint8_t *w, int nb) {
     return (nb & 1) == 0 && ((uintptr_t)w & 3) == 0;
@@ -167,11 +177,11 @@ __global__ __launch_bounds__(64 * Q4_PARTS) void k_q4_vec(Q4Mats mats, const flo
     const uint8_t *wr = mat.w + (size_t)min(r0 + j, n_out - 1) * ((size_t)nb * Q4_BLOCK);
     const Q4Masks km;
     float acc[NT];
-    int E[NT];
+    int E[NT], top[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         acc[t] = 0.0f;
-        E[t] = 1;
+        E[t] = top[t] = 1;
     }
     for (int c0 = b0; c0 < b1; c0 += 8 * NP) {
         // the activations' loads first (the weights' come from further away), then the weights'
@@ -209,7 +219,7 @@ __global__ __launch_bounds__(64 * Q4_PARTS) void k_q4_vec(Q4Mats mats, const flo
         }
         __builtin_amdgcn_sched_barrier(0);
         // x: lane l takes elements 4 (l % 8) .. + 3 of block l / 8 of each pass
-        int ev[NP][NT];  // the largest exponent up to this lane's block
+        int ev[NP][NT], own[NP][NT];  // the largest exponent up to this lane's block, and the block's
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -219,7 +229,8 @@ __global__ __launch_bounds__(64 * Q4_PARTS) void k_q4_vec(Q4Mats mats, const flo
                 mx = maxf_bits(mx, dpp<0xb1>(__builtin_bit_cast(uint32_t, mx)));
                 mx = maxf_bits(mx, dpp<0x4e>(__builtin_bit_cast(uint32_t, mx)));
                 mx = maxf_bits(mx, dpp<0x141>(__builtin_bit_cast(uint32_t, mx)));
-                int e = max(exp_field(mx), E[t]);  // over the 8 blocks of the pass, then those before
+                own[u][t] = exp_field(mx);
+                int e = max(own[u][t], top[t]);  // over the 8 blocks of the pass, then those before
                 e = max(e, __builtin_amdgcn_update_dpp(0, e, 0x118, 0xf, 0xf, false));  // row_shr:8
                 e = max(e, __builtin_amdgcn_update_dpp(0, e, 0x142, 0xa, 0xf, false));  // row_bcast:15
                 ev[u][t] = max(e, __builtin_amdgcn_update_dpp(0, e, 0x143, 0xc, 0xf, false));  // row_bcast:31
@@ -230,7 +241,9 @@ __global__ __launch_bounds__(64 * Q4_PARTS) void k_q4_vec(Q4Mats mats, const flo
             if (c0 == b0) E[t] = __builtin_amdgcn_readlane(ev[0][t], 0);  // nothing to rescale yet
 #pragma unroll
             for (int u = 0; u < NP; ++u) {
-                if (u > 0) ev[u][t] = max(ev[u][t], __builtin_amdgcn_readlane(ev[u - 1][t], 63));
+                if (u > 0) ev[u][t] = max(ev[u][t], top[t]);
+                top[t] = __builtin_amdgcn_readlane(ev[u][t], 63);
+                ev[u][t] = q4_exponent(own[u][t], ev[u][t]);
                 const int s = 141 - ev[u][t];
                 const float4 f = xv[u][t];
                 uint32_t h0, l0, h1, l1;  // elements 0 and 2, 1 and 3
@@ -270,31 +283,42 @@ __global__ __launch_bounds__(64 * Q4_PARTS) void k_q4_vec(Q4Mats mats, const flo
             rows_transpose(nib[0]);
             rows_transpose(nib[1]);
             rows_gather(s, ds);
-            // the pass's blocks, with a look at the exponents before each where one grows inside the pass
-            auto pass = [&](auto growc) {
+            // the pass's blocks, with a look at the exponents before each where one changes inside the pass
+            auto pass = [&](auto changec) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    if constexpr (decltype(growc)::value)
+                for (int i0 = 0; i0 < 8; i0 += 4) {
+                    f16x8 xh[4], wf[4];
+                    f32x4 c[4];
 #pragma unroll
-                        for (int t = 0; t < NT; ++t) {
-                            const int e = __builtin_amdgcn_readlane(ev[u][t], 8 * i);
-                            acc[t] = ldexpf(acc[t], E[t] - e);
-                            E[t] = e;
-                        }
-                    const uint4 *xq = (const uint4 *)(xr + (8 * u + i) * 32);
-                    const f16x8 xh = __builtin_bit_cast(f16x8, xq[0]), xl = __builtin_bit_cast(f16x8, xq[4]);
-                    const f16x8 wf = q4_f16(nib[i & 1][i >> 1], km);
-                    f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, wf, f32x4{0, 0, 0, 0}, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, wf, c, 0, 0, 0);
-                    const f16x2 d = as_f16x2(ds[i >> 1]);
+                    for (int i = 0; i < 4; ++i) {
+                        const uint4 *xq = (const uint4 *)(xr + (8 * u + i0 + i) * 32);
+                        xh[i] = __builtin_bit_cast(f16x8, xq[0]);
+                        wf[i] = q4_f16(nib[i & 1][(i0 + i) >> 1], km);
+                        c[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xq[4]), wf[i],
+                                                                      f32x4{0, 0, 0, 0}, 0, 0, 0);
+                    }
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) acc[t] = fmaf((float)(i & 1 ? d.y : d.x), c[t], acc[t]);
+                    for (int i = 0; i < 4; ++i)
+                        c[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[i], wf[i], c[i], 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        if constexpr (decltype(changec)::value)
+#pragma unroll
+                            for (int t = 0; t < NT; ++t) {
+                                const int e = __builtin_amdgcn_readlane(ev[u][t], 8 * (i0 + i));
+                                acc[t] = ldexpf(acc[t], E[t] - e);
+                                E[t] = e;
+                            }
+                        const f16x2 d = as_f16x2(ds[(i0 + i) >> 1]);
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) acc[t] = fmaf((float)(i & 1 ? d.y : d.x), c[i][t], acc[t]);
+                    }
                 }
             };
-            bool grow = false;
+            bool change = false;
 #pragma unroll
-            for (int t = 0; t < NT; ++t) grow |= __builtin_amdgcn_readlane(ev[u][t], 63) != E[t];
-            if (grow) pass(std::true_type{});
+            for (int t = 0; t < NT; ++t) change |= __builtin_amdgcn_ballot_w64(ev[u][t] != E[t]) != 0;
+            if (change) pass(std::true_type{});
             else pass(std::false_type{});
         }
     }
@@ -335,12 +359,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
     const Q4Masks km;
     f32x4 acc[RT][TT];
-    int E[TT];      // token j's exponent
-    float lim[TT];  // what would raise it
+    // token j's exponent, and what a float in [2^-16, 2) times its power of two exceeds by less than 17 << 23 as
+    // bits; where E is a far block's, a value that every float exceeds by more, with the part's largest exponent
+    // in its low byte
+    int E[TT];
+    uint32_t low[TT];
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
         E[tt] = 1;
-        lim[tt] = __uint_as_float(2u << 23);
+        low[tt] = (uint32_t)(1 - Q4_NEAR) << 23;
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) acc[rt][tt] = f32x4{0, 0, 0, 0};
     }
@@ -379,22 +406,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         for (int i = 0; i < 4; ++i) {
             const int b = c0 + i;
             if (b >= b1) break;
-            // x of the block: its largest against the token's limit, then the split
+            // x of the block: its largest against the token's exponent, then the split
             f16x8 xh[TT], xl[TT];
 #pragma unroll
             for (int tt = 0; tt < TT; ++tt) {
                 const float *lo = xb[i % PB][tt][0].v, *hi = xb[i % PB][tt][1].v;
                 float mx = fmaxf(fmaxf(fmaxf(fabsf(lo[0]), fabsf(lo[1])), fmaxf(fabsf(lo[2]), fabsf(lo[3]))),
                                  fmaxf(fmaxf(fabsf(hi[0]), fabsf(hi[1])), fmaxf(fabsf(hi[2]), fabsf(hi[3]))));
-                if (__builtin_amdgcn_ballot_w64(mx >= lim[tt])) {
+                if (__builtin_amdgcn_ballot_w64(__float_as_uint(mx) - low[tt] >= (Q4_NEAR + 1u) << 23)) {
                     mx = fmaxf(mx, __shfl_xor(mx, 16));
                     mx = fmaxf(mx, __shfl_xor(mx, 32));
-                    const int e = max(E[tt], exp_field(mx)), grow = E[tt] - e;
+                    const int own = exp_field(mx), far = low[tt] & 0xFF, top = max(far ? far : E[tt], own);
+                    const int e = q4_exponent(own, top), change = E[tt] - e;
                     E[tt] = e;
-                    lim[tt] = __uint_as_float((uint32_t)min(e + 1, 255) << 23);
+                    low[tt] = e == top ? (uint32_t)(e - Q4_NEAR) << 23 : 0x80000000u | (uint32_t)top;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        const int by = __shfl(grow, 4 * g + r);
+                        const int by = __shfl(change, 4 * g + r);
 #pragma unroll
                         for (int rt = 0; rt < RT; ++rt) acc[rt][tt][r] = ldexpf(acc[rt][tt][r], by);
                     }

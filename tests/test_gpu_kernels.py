@@ -498,3 +498,51 @@ def test_q4_mm_many_rows_token_counts_share_their_bits(gpu, n_out, k, offset):
     for n in ns:
         print(f"[q4] {n_out} x {k}, {n} tokens", flush=True)
         assert np.array_equal(run(0, n), one[:n], equal_nan=True), n
+
+
+@pytest.mark.parametrize("n_out,k", [(200, 2816), (257, 2720), (9000, 256), (2100, 640)])
+def test_q4_mm_activation_blocks_far_apart(gpu, n_out, k):
+    """rvh_q4_mm under 16384 rows where a token's blocks lie up to 2^40 apart and the weights of the large ones
+    are 0 or as much smaller, so that the small ones carry the rows: each token within the operator's bound
+    (relative L2 1e-5) of the exact product. Tokens whose blocks' exponents jump by up to 2^90 either way, some of
+    them zeros or subnormal values, have the bits of their call alone in every call."""
+    rng = np.random.default_rng(n_out + k)
+    nb = k // 32
+    steps = [0, 13, 17, 20, 26, 40]
+    large = np.arange(nb) % 3 == 0
+    for dscale in (0.0, 1.0):
+        w = rand_q4(rng, n_out, k, 0.01, 0.03)
+        blk = w.reshape(n_out, nb, 18)
+        blk[:, large, :2] = np.full(1, 2.0 ** -18 * dscale, np.float16).view(np.uint8)
+        wf = dequant_q4(w, n_out, k).astype(np.float64)
+        x = rng.standard_normal((len(steps), nb, 32)).astype(np.float32)
+        for t, s in enumerate(steps):
+            x[t, large] *= np.float32(2.0 ** (min(s, 17) if dscale else s))
+        x = x.reshape(-1, k)
+        want = x.astype(np.float64) @ wf.T
+        for n_in in (1, 4, len(steps), 4 * len(steps)):
+            print(f"[q4] far {n_out} x {k}, {n_in} tokens", flush=True)
+            for t0 in range(0, len(steps), n_in):
+                xs = np.concatenate([x] * 5)[t0:t0 + n_in]
+                y = DevBuf(n_in * n_out * 4)
+                hip.q4_mm(dev(w), dev(xs), y, n_out, k, n_in)
+                got = y.download(np.float32, n_in * n_out).reshape(n_in, n_out).astype(np.float64)
+                ref = np.concatenate([want] * 5)[t0:t0 + n_in]
+                err = np.sqrt(((got - ref) ** 2).sum(1) / (ref ** 2).sum(1))
+                assert err.max() < 1e-5, (dscale, n_in, steps[int(err.argmax() + t0) % len(steps)], err.max())
+    ns = [2, 3, 4, 5, 16, 17, 40]
+    x = rng.standard_normal((max(ns), nb, 32)) * 2.0 ** rng.integers(-45, 46, (max(ns), nb, 1))
+    x[rng.random((max(ns), nb)) < 0.2] = 0.0
+    x[rng.random((max(ns), nb)) < 0.1] *= 2.0 ** -130
+    x[3], x[20, 5:] = 0.0, 0.0
+    x = x.reshape(-1, k).astype(np.float32)
+    w = dev(rand_q4(rng, n_out, k, 0.01, 0.03))
+    y = DevBuf(max(ns) * n_out * 4)
+
+    def run(xs):
+        hip.q4_mm(w, dev(xs), y, n_out, k, len(xs))
+        return y.download(np.float32, len(xs) * n_out).reshape(len(xs), n_out).copy()
+
+    one = np.concatenate([run(x[t:t + 1]) for t in range(max(ns))])
+    for n in ns:
+        assert np.array_equal(run(x[:n]), one[:n]), n
