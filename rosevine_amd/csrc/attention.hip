@@ -1696,10 +1696,35 @@ int launch_stream(const float *q, const void *kc, const void *vc, float *out, fl
 // 1244 / 247; hd 128, 2 x 4 x 512 13.8 / 14.1, 2 x 2 x 4002 25.0 / 18.0, 400 x 2 x 3400 1323 / 87; hd 64,
 // 2 x 4 x 4002 23.4 / 14.0, 400 x 4 x 3400 1329 / 32. Four waves a workgroup for hd 128 (two workgroups
 // per CU: 87 us against 98 with eight), eight for the others (hd 64: 32 against 42 with four).
-inline bool attn_prefill_ok(int n_tok, int n_head, int n_kv, int hd, int p0, int window) {
-    const long keys = (long)n_tok * n_kv * attn_longest(n_tok, p0, window);
-    return n_tok > 1 && (hd == 64 || hd == 128 || hd == 256 || hd == 512) && keys >= (hd > 256 ? 40000 : hd > 128 ? 64000 : 12000) &&
-           (long)n_tok * n_head <= 0x7fffffffL - 64 && (long)n_kv * (hd / QK * Q8_BLOCK) * PF_KEYS <= 0x7fffffffL;
+//
+// Several chunks shorten the per-token kernels' chains, so there the line lies higher (tokens x heads x keys in
+// chunks, merged):
+//  - hd 64 and 128: by rows x keys, as the per-token kernel computes every head apart, and further up where
+//    its tiles of 64 keys are full: hd 128, 2 x 8 heads x 766 keys in 12 chunks 9.1 / 11.2, in 24 10.6 / 11.0,
+//    16 x 4 x 376 in 6 10.7 / 11.5, 4 x 8 x 1024 in 16 10.8 / 11.1, 2 x 16 x 766 in 24 12.2 / 11.3; hd 64,
+//    16 x 8 x 96 in 2 9.2 / 10.2, 2 x 8 x 1024 in 32 10.5 / 9.3;
+//  - two tokens of at most two heads per kv head are 4 of 32 rows, and where they make more workgroups than CUs
+//    the per-token kernel's shorter ones win: hd 128, 2 x 8 x 2251 in 36 12.4 / 14.4; hd 64 12.2 / 14.9 (but
+//    hd 128, 2 x 8 x 4001 in 126 22.8 / 20.1);
+//  - hd 256 and 512, four heads and more per kv head: k_attn_stream takes them at the price of one, and where its
+//    grid just fits the CUs it is at its best: hd 256, 16 x 16 heads x 1021 keys in 4 chunks 21.8 / 25.3, x 1401
+//    25.8 / 27.2 (in 8 chunks 30.8 / 22.8); hd 512, 16 x 8 x 1276 in 8 25.5 / 28.8 (in 16 33.7 / 25.1).
+inline bool attn_prefill_ok(int n_tok, int n_head, int n_kv, int hd, int p0, int window, int n_chunks) {
+    const long longest = attn_longest(n_tok, p0, window), keys = (long)n_tok * n_kv * longest;
+    if (n_tok < 2 || (hd != 64 && hd != 128 && hd != 256 && hd != 512) ||
+        keys < (hd > 256 ? 40000 : hd > 128 ? 64000 : 12000) || (long)n_tok * n_head > 0x7fffffffL - 64 ||
+        (long)n_kv * (hd / QK * Q8_BLOCK) * PF_KEYS > 0x7fffffffL)
+        return false;
+    if (n_chunks == 1) return true;
+    const int per_kv = n_head / n_kv, cus = device_cus();
+    if (hd > 128) {
+        const long wgs = (long)n_tok * n_kv * n_chunks;  // of k_attn_stream
+        return per_kv < 4 || wgs > cus || wgs <= cus / 2 || keys >= (hd > 256 ? 60000 : 96000);
+    }
+    const long work = (long)n_tok * n_head * longest;
+    const bool full = longest > 32L * n_chunks;  // chunks of more than half a tile of k_attn_split
+    if (work < (hd == 64 ? (full ? 16500 : 12000) : (full ? 30000 : 16500))) return false;
+    return n_tok > 2 || per_kv > 2 || (long)n_kv * n_chunks <= cus || work >= 50000;
 }
 
 template <int NBW, int TW, int WV>
@@ -1714,7 +1739,7 @@ int launch_prefill(const float *q, const uint8_t *kc, const uint8_t *vc, float *
 
 int launch_attn(const float *q, const void *kc, const void *vc, float *out, float *part, int n_tok, int n_head,
                 int n_kv, int hd, int p0, int cap, int window, int n_chunks) {
-    if (attn_prefill_ok(n_tok, n_head, n_kv, hd, p0, window)) {
+    if (attn_prefill_ok(n_tok, n_head, n_kv, hd, p0, window, n_chunks)) {
         const uint8_t *k8 = (const uint8_t *)kc, *v8 = (const uint8_t *)vc;
 #define RVM_PREFILL_ARGS q, k8, v8, out, part, n_tok, n_head, n_kv, p0, cap, window, n_chunks
         if (hd == 512) return launch_prefill<4, 4, 8>(RVM_PREFILL_ARGS);

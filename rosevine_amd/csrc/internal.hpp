@@ -385,6 +385,7 @@ inline int with_steps(int n, F &&f) {
 
 // Device limits read once per process (rvh_init).
 int max_lds_per_block();
+int device_cus();  // the current device's CUs (256 where it cannot be asked)
 // The per-device address of rvm_moe_decode_static's scratch array, taken once per device with
 // that device current (decode.hip; rvh_init calls it).
 int static_scratch_setup(int device);

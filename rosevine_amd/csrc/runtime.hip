@@ -2,6 +2,8 @@
 // The rvh_* symbols keep the meaning of the reference's runtime/hip/rvhip.h:22-38
 // (runtime/hip/rvhip.hip:449-509); transfers and events use the library's current stream so that
 // they stay ordered with the kernels issued there.
+#include <atomic>
+
 #include "internal.hpp"
 
 namespace rvm {
@@ -46,6 +48,17 @@ int launched() {
 
 // LDS a workgroup may allocate on the current device, capped at the 64 KiB that needs no
 // per-kernel attribute.
+int device_cus() {
+    static std::atomic<int> cache[64];
+    int dev = 0, x = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if ((x = cache[dev].load(std::memory_order_relaxed)) == 0) {
+        if (hipDeviceGetAttribute(&x, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || x < 1) return 256;
+        cache[dev].store(x, std::memory_order_relaxed);
+    }
+    return x;
+}
+
 int max_lds_per_block() {
     static int v = 0;
     if (!v) {
