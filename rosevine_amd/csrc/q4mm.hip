@@ -940,15 +940,21 @@ inline bool q4_uses_i8(int n_out, int k) { return n_out >= QI_MIN_ROWS && k / QK
 int q4_run_i8(const uint8_t *w, const float *x, float *y, int n_out, int k, int n_in) {
     const int nb = k / QK;
     const bool aln = q4_rows_aligned(w, nb);
-    // From 5 tokens (3 on rows that are not on dwords) 8, 16 or 32 a pass over the matrix, and the more rows
-    // a workgroup shares its digits with the fewer workgroups: 262,144 x 2816, 32 tokens: 32 x 8 rows a
-    // workgroup 321 us, 64 x 8 254 (eight passes of 4 tokens 897); 8 tokens 112 / 120 (228); 100,000 x 2080
-    // unaligned, 4 tokens: 67 in a pass of 4, 57 here; 40,001 x 4096, 4 tokens: 42 in a pass of 4, 47 here.
-    // 16, 32 and 64 rows a wave, 32 tokens: 20,000 x 2816 51 / 78 / -, 40,001 x 4096 164 / 108 / -, 70,000 x
-    // 2816 - / 155 / 124, 100,000 x 2816 - / 155 / 124.
-    if (n_in > (aln ? 4 : 2)) {
-        const int nq = n_in <= 8 ? 2 : n_in <= 16 ? 4 : 8;
-        const int rt = n_out >= 65536 && nq == 8 ? 4 : n_out >= 32768 ? 2 : 1;
+    // From 5 tokens (3 on rows that are not on dwords) 8, 16 or 32 a pass over the matrix: 262,144 x 2816, 32
+    // tokens 254 us (eight passes of 4 tokens 897), 8 tokens 120 (228); 100,000 x 2080 unaligned, 4 tokens:
+    // 67 in a pass of 4, 57 here; 40,001 x 4096, 4 tokens: 42 in a pass of 4, 47 here. Two tokens a pass (where
+    // four tokens' digits do not fit 64 KB) still win while all passes are two workgroups a CU: 16,384 x 4096,
+    // 5 tokens 27 / 32, 8 tokens 29 / 32; 20,000 rows 30 / 33 and 44 / 33.
+    const int cus = device_cus(), tt = qi_tokens(nb, n_in), tiles = grid_blocks(n_out, QI_WAVES * 16);
+    if (n_in > (aln ? 4 : 2) && !(aln && tt == 2 && (long)tiles * grid_blocks(n_in, 2) <= 2L * cus)) {
+        // Half the tokens a pass while the CUs take both passes at once: 16,384 x 2816, 9 tokens 28 us in a pass
+        // of 16, 20 in two of 8; 32 tokens 52 in a pass of 32, 28 in two of 16. Then 16 rows a wave while
+        // those workgroups fit the CUs, and 32 (64 for 32 tokens) as long: the more rows a workgroup shares its digits
+        // with the longer it takes, 52 / 75 / 122 us a round at 32 tokens and k 2816 (32,768 rows 52 / 76 / 123;
+        // 65,536 83 / 77 / 124; 100,000 154 / 149 / 124).
+        int nq = n_in <= 8 ? 2 : n_in <= 16 ? 4 : 8;
+        while (nq > 2 && (long)tiles * grid_blocks(n_in, 2 * nq) <= cus) nq >>= 1;
+        const int rt = tiles <= cus ? 1 : nq == 8 && tiles > 2 * cus ? 4 : 2;
         RVM_CHECK(grid_blocks(n_in, 4 * nq) <= 65535);
         const dim3 grid(grid_blocks(n_out, QI_WAVES * 16 * rt), grid_blocks(n_in, 4 * nq));
         auto go = [&](auto kern) {
@@ -970,7 +976,6 @@ int q4_run_i8(const uint8_t *w, const float *x, float *y, int n_out, int k, int 
         else by_rows(std::integral_constant<int, 8>{});
         return launched();
     }
-    const int tt = qi_tokens(nb, n_in);
     const dim3 grid(grid_blocks(n_out, QI_WAVES * QI_ROWS), grid_blocks(n_in, tt));
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, grid, dim3(QI_WAVES * 64), qi_lds_bytes(nb, tt), cur_stream(), w, x, y, n_out, k, n_in);

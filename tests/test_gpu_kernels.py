@@ -468,6 +468,8 @@ def test_q4_mm_activation_edge_cases(gpu, n_in):
 
 
 @pytest.mark.parametrize("n_out,k,offset", [
+    (16384, 352, 0),    # 128 workgroups: half the tokens a pass from 9 to 16 and 17 to 32
+    (16384, 4160, 0),   # two tokens a pass up to 8
     (16389, 96, 0),     # 16 rows a wave, 3 blocks: unaligned, one chunk of 8 with 5 past the row
     (16400, 2816, 2),   # the matrix 2 bytes past a dword
     (33001, 320, 0),    # 32 rows a wave
