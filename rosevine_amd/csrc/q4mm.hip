@@ -165,14 +165,23 @@ __device__ __forceinline__ Q4Mat q4_matrix(const Q4Mats &mats, int bx) {
 // 24.0 with f32 products on the VALU; 4 tokens 29.8 / 41.5; loads under branches took 25.1).
 constexpr int QV_CH = 4;  // passes of 8 blocks in registers at most
 
-template <int NT, int NP, bool ALN>  // tokens; the part's passes of 8 blocks, at most QV_CH at once
+// How a lane loads its two blocks: as two, where the matrix starts on 2 bytes or its rows are one block; as 9
+// dwords, where every pair starts on one; shifted, as the dwords that hold the 36 bytes (a pair 2 bytes past a
+// dword ends in the low half of the last one, which is loaded as such). Two blocks at 2-byte addresses cost a
+// row of 65 blocks half a microsecond and more (1 token, 1000 x 2080: 5.3 us, shifted 5.1; one layer's seven
+// projections on odd block counts 29.2 / 26.6).
+enum { QV_SPLIT, QV_DWORDS, QV_SHIFTED };
+
+template <int NT, int NP, int LD>  // tokens a pass (blockIdx.y); the part's passes of 8 blocks, at most QV_CH at once
 __global__ __launch_bounds__(64 * Q4_PARTS) void k_q4_vec(Q4Mats mats, const float *__restrict__ x, int k, int n_in) {
     __shared__ __attribute__((aligned(16))) uint32_t xs[Q4_PARTS][NT][NP * 8 * 32];  // [block][hi, lo][g][4]
     __shared__ float ps[Q4_PARTS][NT][16];
     const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
     const int p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Q4Mat mat = q4_matrix(mats, blockIdx.x);
-    const int n_out = mat.n_out, r0 = mat.wg * 16;
+    const int n_out = mat.n_out, r0 = mat.wg * 16, t0 = blockIdx.y * NT;
+    x += (size_t)t0 * k;
+    n_in -= t0;
     const int nb = k / QK, qb = q4_part(nb), b0 = p * qb, b1 = min(nb, b0 + qb);
     const uint8_t *wr = mat.w + (size_t)min(r0 + j, n_out - 1) * ((size_t)nb * Q4_BLOCK);
     const Q4Masks km;
@@ -197,8 +206,9 @@ __global__ __launch_bounds__(64 * Q4_PARTS) void k_q4_vec(Q4Mats mats, const flo
 #pragma unroll
         for (int u = 0; u < NP; ++u) {
             const int b = c0 + 8 * u + 2 * g;
-            if constexpr (ALN) {
-                const uint8_t *a = wr + min(b, nb - 2) * Q4_BLOCK;
+            if constexpr (LD != QV_SPLIT) {
+                const uint8_t *p = wr + min(b, nb - 2) * Q4_BLOCK;
+                const uint8_t *a = LD == QV_SHIFTED ? (const uint8_t *)((uintptr_t)p & ~(uintptr_t)3) : p;
                 const Dwords<4> d0 = *(const Dwords<4> *)a, d1 = *(const Dwords<4> *)(a + 16);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -206,6 +216,7 @@ __global__ __launch_bounds__(64 * Q4_PARTS) void k_q4_vec(Q4Mats mats, const flo
                     v[u][4 + i] = d1.q[i];
                 }
                 v[u][8] = *(const uint32_t *)(a + 32);
+                if constexpr (LD == QV_SHIFTED) v[u][9] = *(const uint16_t *)(p + 34);
             } else {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -262,13 +273,23 @@ __global__ __launch_bounds__(64 * Q4_PARTS) void k_q4_vec(Q4Mats mats, const flo
         for (int u = 0; u < NP; ++u) {
             if (c0 + 8 * u >= b1) break;
             uint32_t nib[2][4], ds[4], s;
-            if constexpr (ALN) {
+            if constexpr (LD != QV_SPLIT) {
+                if constexpr (LD == QV_SHIFTED) {
+                    const uint32_t by = (uintptr_t)(wr + min(c0 + 8 * u + 2 * g, nb - 2) * Q4_BLOCK) & 2;
+#pragma unroll
+                    for (int i = 0; i < 9; ++i) v[u][i] = __builtin_amdgcn_alignbyte(v[u][i + 1], v[u][i], by);
+                }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     nib[0][i] = __builtin_amdgcn_perm(v[u][i + 1], v[u][i], 0x05040302u);
                     nib[1][i] = v[u][5 + i];
                 }
                 s = __builtin_amdgcn_perm(v[u][4], v[u][0], 0x07060100u);
+                if (LD == QV_SHIFTED && c0 + 8 * u + 2 * g == nb - 1) {  // a row's last block, loaded behind another
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) nib[0][i] = nib[1][i];
+                    s >>= 16;
+                }
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -328,7 +349,7 @@ __global__ __launch_bounds__(64 * Q4_PARTS) void k_q4_vec(Q4Mats mats, const flo
     __syncthreads();
     const int r = threadIdx.x & 15, t = threadIdx.x >> 4;
     if (t < NT && t < n_in && r0 + r < n_out)
-        mat.y[(size_t)t * n_out + r0 + r] = (ps[0][t][r] + ps[1][t][r]) + (ps[2][t][r] + ps[3][t][r]);
+        mat.y[(size_t)(t0 + t) * n_out + r0 + r] = (ps[0][t][r] + ps[1][t][r]) + (ps[2][t][r] + ps[3][t][r]);
 }
 
 // ---- Several tokens. A workgroup of four waves takes 16 RT rows x 16 TT tokens, wave p part p of the
@@ -891,23 +912,36 @@ int q4_run(Q4Mats &mats, const float *x, int k, int n_in) {
     if (mats.n == 0) return 0;
     long rows = 0;
     for (int m = 0; m < mats.n; ++m) rows += mats.n_out[m];
-    // Up to four tokens, each its own conversion in the wave (5 tokens: 40 us a layer's seven products
-    // against 43 here), then 16 to a tile.
-    if (n_in <= 4) {
-        bool aln = true;
-        for (int m = 0; m < mats.n; ++m) aln = aln && q4_rows_aligned(mats.w[m], k / QK);
-        const long wgs = q4_starts(mats, 1);
-        RVM_CHECK(wgs > 0);
+    bool dwords = true, shifted = k / QK > 1;
+    for (int m = 0; m < mats.n; ++m) {
+        dwords = dwords && q4_rows_aligned(mats.w[m], k / QK);
+        shifted = shifted && ((uintptr_t)mats.w[m] & 3) == 0;
+    }
+    const int cus = device_cus();
+    // Up to four tokens a pass, each its own conversion in the wave (5 tokens: 40 us a layer's seven products
+    // against 43 here), and more passes while they are two workgroups a CU (one for few tokens on rows that are not
+    // on dwords): a tile's parts are longer chains. 5 tokens, 1000 x 4096 14 us in a tile, 8 here (8 f32
+    // products on the VALU), 33 tokens, 512 x 2816 17 / 9; 4096 x 2816, 5 tokens 9.1 / 8.7, 8 of 8192 rows
+    // 9.7 / 13; 4096 x 2080, 5 tokens 8.5 / 9.4.
+    const long vec_wgs = q4_starts(mats, 1), passes = grid_blocks(n_in, 4);
+    RVM_CHECK(vec_wgs > 0);
+    if (n_in <= 4 || vec_wgs * passes <= (dwords || n_in > 16 ? 2L : 1L) * cus) {
         auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * Q4_PARTS), 0, cur_stream(), mats, x, k, n_in);
+            hipLaunchKernelGGL(kern, dim3((unsigned)vec_wgs, (unsigned)passes), dim3(64 * Q4_PARTS), 0, cur_stream(),
+                               mats, x, k, n_in);
+        };
+        auto by_loads = [&](auto ntc, auto npc) {
+            constexpr int NT = decltype(ntc)::value, NP = decltype(npc)::value;
+            if (dwords) go(k_q4_vec<NT, NP, QV_DWORDS>);
+            else if (shifted) go(k_q4_vec<NT, NP, QV_SHIFTED>);
+            else go(k_q4_vec<NT, NP, QV_SPLIT>);
         };
         auto by_passes = [&](auto ntc) {
-            constexpr int NT = decltype(ntc)::value;
             switch (min(QV_CH, grid_blocks(q4_part(k / QK), 8))) {
-                case 1: aln ? go(k_q4_vec<NT, 1, true>) : go(k_q4_vec<NT, 1, false>); break;
-                case 2: aln ? go(k_q4_vec<NT, 2, true>) : go(k_q4_vec<NT, 2, false>); break;
-                case 3: aln ? go(k_q4_vec<NT, 3, true>) : go(k_q4_vec<NT, 3, false>); break;
-                default: aln ? go(k_q4_vec<NT, 4, true>) : go(k_q4_vec<NT, 4, false>); break;
+                case 1: by_loads(ntc, std::integral_constant<int, 1>{}); break;
+                case 2: by_loads(ntc, std::integral_constant<int, 2>{}); break;
+                case 3: by_loads(ntc, std::integral_constant<int, 3>{}); break;
+                default: by_loads(ntc, std::integral_constant<int, 4>{}); break;
             }
         };
         if (n_in == 1) by_passes(std::integral_constant<int, 1>{});
@@ -915,15 +949,16 @@ int q4_run(Q4Mats &mats, const float *x, int k, int n_in) {
         else by_passes(std::integral_constant<int, 4>{});
         return launched();
     }
+    // Then tiles of 16 tokens, or 32.
     const int tt = n_in > 16 ? 2 : 1, ty = grid_blocks(n_in, 16 * tt);
     RVM_CHECK(ty <= 65535);
-    // The largest tile of which there are still 140, over half the CUs: a larger tile converts each x and
-    // each nibble for more products, which outweighs idle CUs until about there. One layer's seven
+    // The largest tile of which there are still 35/64 of the CUs (140 of 256): a larger tile converts each x
+    // and each nibble for more products, which outweighs idle CUs until about there. One layer's seven
     // projections, at least 512 / 220 / 140 / 110 workgroups: 250 tokens 189 / 168 / 152 / 152 us, 100
     // tokens 137 / 122 / 100 / 99, 16 tokens 47.7 / 47.7 / 47.8 / 50.8; 500 tokens at width 1024 123 / 104 /
     // 104 / 117.
     int rt = 8;
-    while (rt > 2 && (rows + 16 * rt - 1) / (16 * rt) * ty < 140) rt >>= 1;
+    while (rt > 2 && (rows + 16 * rt - 1) / (16 * rt) * ty < 35L * cus / 64) rt >>= 1;
     const long wgs = q4_starts(mats, rt);
     RVM_CHECK(wgs > 0);
     auto go = [&](auto kern) {

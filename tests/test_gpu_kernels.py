@@ -408,6 +408,8 @@ def test_q4_mm_n_equals_one_call_per_matrix(gpu, rows, k):
     (1030, 2816, 2),   # a matrix 2 bytes past a dword
     (95, 4160, 0),     # 130 blocks: parts of more than four passes
     (9000, 256, 0),    # the 64- and 128-row tiles
+    (2110, 160, 0),    # the 32-row tiles; passes of four tokens below
+    (1009, 608, 2),    # an odd block count 2 bytes past a dword
 ])
 def test_q4_mm_token_counts_share_their_bits(gpu, orc, n_out, k, offset):
     """rvh_q4_mm under 16384 rows at the edges of its token tiles: every token of a call has the bits of
@@ -416,7 +418,7 @@ def test_q4_mm_token_counts_share_their_bits(gpu, orc, n_out, k, offset):
     w = rand_q4(rng, n_out, k, 0.01, 0.03)
     wd = DevBuf(w.nbytes + 2)
     wd.upload(w, offset)
-    ns = [2, 3, 4, 5, 16, 17, 33, 130]
+    ns = [2, 3, 4, 5, 16, 17, 33, 130, 300]
     x = (rng.standard_normal((max(ns), k)) * 10.0 ** rng.uniform(-3, 3, (max(ns), 1))).astype(np.float32)
     xd, y = dev(x), DevBuf(max(ns) * n_out * 4)
 
