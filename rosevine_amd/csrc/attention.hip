@@ -34,7 +34,6 @@ constexpr int AT_MAXHD = 512;  // dimensions per head (8 per lane)
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef int v2i_t __attribute__((ext_vector_type(2)));
 
 struct __attribute__((packed, aligned(2))) Q8Half {  // 8 quants of a Q8_0 block
@@ -836,8 +835,6 @@ __device__ __forceinline__ uint32_t pf_near_bits(int E) {
     return e >= -14 ? (uint32_t)(e + 15) << 10 : e >= -24 ? 1u << (e + 24) : 1u;
 }
 
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 template <int NBW, int TW, int WV>
@@ -870,12 +867,6 @@ __device__ __forceinline__ void loads_left() {  // at most N vector memory opera
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
 
-__device__ __forceinline__ f16x2 as_f16x2(uint32_t u) { return __builtin_bit_cast(f16x2, u); }
-__device__ __forceinline__ uint32_t as_u32(f16x2 h) { return __builtin_bit_cast(uint32_t, h); }
-__device__ __forceinline__ f16x8 as_f16x8(const uint32_t *u) {
-    return __builtin_bit_cast(f16x8, uint4{u[0], u[1], u[2], u[3]});
-}
-
 // eight int8 quants as f16: 0x6400 | (q + 128) is 1152 + q
 __device__ __forceinline__ f16x8 q8x8_f16(uint32_t a, uint32_t b) {
     const f16x2 off = {(_Float16)1152.0f, (_Float16)1152.0f};
@@ -887,14 +878,6 @@ __device__ __forceinline__ f16x8 q8x8_f16(uint32_t a, uint32_t b) {
     u[2] = as_u32(as_f16x2(__builtin_amdgcn_perm(0x64646464u, b, 0x04010400u)) - off);
     u[3] = as_u32(as_f16x2(__builtin_amdgcn_perm(0x64646464u, b, 0x04030402u)) - off);
     return as_f16x8(u);
-}
-
-// x = hi + lo in f16 (rounded, then the exact residual rounded); an infinite x leaves lo = NaN
-__device__ __forceinline__ void split2_f16(float x0, float x1, f16x2 &hi, f16x2 &lo) {
-    float neg1 = -1.0f;
-    asm("" : "+s"(neg1));  // unknown to the compiler, so that each residual stays one v_fma_mix_f32
-    hi = __builtin_convertvector((f32x2{x0, x1}), f16x2);
-    lo = __builtin_convertvector((f32x2{fmaf((float)hi.x, neg1, x0), fmaf((float)hi.y, neg1, x1)}), f16x2);
 }
 
 struct __attribute__((packed, aligned(4))) F4u {  // four floats on any dword
@@ -1039,10 +1022,6 @@ __global__ __launch_bounds__(WV * 64) void k_attn_prefill(
                 }
                 qh[b][m] = as_f16x8(hi);
                 ql[b][m] = as_f16x8(lw);
-                if constexpr (NBW == 8) {  // in accumulation registers: only MFMAs read them
-                    asm("" : "+a"(qh[b][m]));
-                    asm("" : "+a"(ql[b][m]));
-                }
             }
             if (b % 2) __builtin_amdgcn_sched_barrier(0);
         }

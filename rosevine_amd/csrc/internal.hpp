@@ -216,26 +216,22 @@ __device__ __forceinline__ uint32_t swz_xor16(uint32_t v) {
 }
 __device__ __forceinline__ float maxf_bits(float a, uint32_t b) { return fmaxf(a, __builtin_bit_cast(float, b)); }
 
-// a & m, opaque to the optimiser: byte conversions of the result then map to v_cvt_f32_ubyte0..3,
-// one instruction each, where knowing the bytes are nibbles makes the compiler extract each one
-// first.
-__device__ __forceinline__ uint32_t and_opaque(uint32_t a, uint32_t m) {
-    uint32_t r;
-    asm("v_and_b32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(m));
-    return r;
+// f16 pairs: operands of the f16 matrix instructions that stand for f32 values.
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ f16x2 as_f16x2(uint32_t u) { return __builtin_bit_cast(f16x2, u); }
+__device__ __forceinline__ uint32_t as_u32(f16x2 h) { return __builtin_bit_cast(uint32_t, h); }
+__device__ __forceinline__ f16x8 as_f16x8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    return __builtin_bit_cast(f16x8, uint4{a, b, c, d});
 }
-
-// Sum over the wave in a fixed order: rows of 16 by DPP, then the four rows.
-__device__ __forceinline__ float wave_sum_dpp(float v) {
-    v += __builtin_bit_cast(float, dpp<0xb1>(__builtin_bit_cast(uint32_t, v)));
-    v += __builtin_bit_cast(float, dpp<0x4e>(__builtin_bit_cast(uint32_t, v)));
-    v += __builtin_bit_cast(float, dpp<0x141>(__builtin_bit_cast(uint32_t, v)));
-    v += __builtin_bit_cast(float, dpp<0x140>(__builtin_bit_cast(uint32_t, v)));
-    const float a = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 0));
-    const float b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 16));
-    const float c = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 32));
-    const float d = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 48));
-    return (a + b) + (c + d);
+__device__ __forceinline__ f16x8 as_f16x8(const uint32_t *u) { return as_f16x8(u[0], u[1], u[2], u[3]); }
+// x = hi + lo in f16 (rounded, then the exact residual rounded); an infinite x leaves lo = NaN
+__device__ __forceinline__ void split2_f16(float x0, float x1, f16x2 &hi, f16x2 &lo) {
+    float neg1 = -1.0f;
+    asm("" : "+s"(neg1));  // unknown to the compiler, so that each residual stays one v_fma_mix_f32
+    hi = __builtin_convertvector((f32x2{x0, x1}), f16x2);
+    lo = __builtin_convertvector((f32x2{fmaf((float)hi.x, neg1, x0), fmaf((float)hi.y, neg1, x1)}), f16x2);
 }
 
 // Orders LDS traffic between lanes of one wave (a wave's LDS operations complete in issue order).

@@ -24,9 +24,6 @@
 
 namespace rvm {
 
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
@@ -45,12 +42,6 @@ struct __attribute__((packed, aligned(4))) Floats4 {
 constexpr int Q4_PARTS = 4;
 // Blocks per part: even, so that the parts of a row whose blocks pair up on dwords start on a pair.
 __host__ __device__ constexpr int q4_part(int nb) { return 2 * ((nb + 2 * Q4_PARTS - 1) / (2 * Q4_PARTS)); }
-
-__device__ __forceinline__ uint32_t as_u32(f16x2 h) { return __builtin_bit_cast(uint32_t, h); }
-__device__ __forceinline__ f16x2 as_f16x2(uint32_t u) { return __builtin_bit_cast(f16x2, u); }
-__device__ __forceinline__ f16x8 as_f16x8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
-    return __builtin_bit_cast(f16x8, uint4{a, b, c, d});
-}
 
 // The nibble masks and f16 biases, unknown to the compiler where it would otherwise make two
 // instructions of a masked or.
@@ -72,13 +63,12 @@ __device__ __forceinline__ f16x8 q4_f16(uint32_t w, const Q4Masks &k) {
                     as_u32(__builtin_elementwise_fma(as_f16x2((v & k.hi) | k.one), s, t)));
 }
 
-// x = hi + lo (rounded, then the exact residual rounded); an infinite x leaves lo = NaN
+// split2_f16 with the pairs as dwords
 __device__ __forceinline__ void q4_split(float x0, float x1, uint32_t &hi, uint32_t &lo) {
-    float neg1 = -1.0f;
-    asm("" : "+s"(neg1));  // unknown to the compiler, so that each residual stays one v_fma_mix_f32
-    const f16x2 h = __builtin_convertvector((f32x2{x0, x1}), f16x2);
+    f16x2 h, l;
+    split2_f16(x0, x1, h, l);
     hi = as_u32(h);
-    lo = as_u32(__builtin_convertvector((f32x2{fmaf((float)h.x, neg1, x0), fmaf((float)h.y, neg1, x1)}), f16x2));
+    lo = as_u32(l);
 }
 
 // Lane rows of 16: after swap32, a = (a's rows 0 1, b's 0 1), b = (a's 2 3, b's 2 3); after swap16,
