@@ -746,9 +746,10 @@ int launch_router(const rvm_layer *L, const float *x, int n_tok, int flags, cons
                                    dim3(FW * 64), 0, cur_stream(), L->router, pre ? rin : x, L->router_bias, n_tok,
                                    L->n_exp, R, pre ? nullptr : xq8, pre ? nullptr : xsc);
             };
-            // eight waves from one workgroup per CU: 1999 tokens 113 us with four, 80 with eight
+            // eight waves from one workgroup per CU: 1999 tokens 113 us with four, 80 with eight. Beyond d = 2816 (of
+            // the compiled widths, 4096) eight rows and the two staged chunks, 128 + 64 KB, pass a CU's 160 KB of LDS.
             bool wide = false;
-            if constexpr (F4 <= 11) wide = grid_blocks(L->n_exp, 8) * grid_blocks(n_tok, 64) >= 256;
+            if constexpr (F4 <= 11) wide = grid_blocks(L->n_exp, 8) * grid_blocks(n_tok, 64) >= device_cus();
             if constexpr (F4 <= 11) {
                 if (wide) fold(std::integral_constant<int, 8>{});
             }
