@@ -369,7 +369,7 @@ def test_q4_mm_n_with_a_many_row_matrix(gpu):
     ws = [hip.DevBuf(r * (k // 32) * 18) for r in rows]
     for i, (w, r) in enumerate(zip(ws, rows)):
         hip.synth_q4(w, 1, r, k, 9, 70 + i)
-    for n_in in (1, 2):
+    for n_in in (1, 2, 5, 17, 130):
         x = dev((rng.standard_normal((n_in, k)) * 0.5).astype(np.float32))
         ys = [hip.DevBuf(n_in * r * 4) for r in rows]
         hip.q4_mm_n(ws, x, ys, list(rows), k, n_in)
@@ -384,14 +384,16 @@ def test_q4_mm_n_with_a_many_row_matrix(gpu):
     ((2112, 2112), 2816),         # gate and up
     ((5, 33, 64, 130), 96),       # four matrices, row counts that split workgroups, a short k
     ((1000,), 4096),              # one matrix
+    ((4500, 4500, 4500, 4490), 512),  # enough rows for 128 a workgroup at 16 tokens, which none has alone
 ])
 def test_q4_mm_n_equals_one_call_per_matrix(gpu, rows, k):
-    """rvm_q4_mm_n: each matrix's output is rvh_q4_mm's, bit for bit, for one and for three tokens."""
+    """rvm_q4_mm_n: each matrix's output is rvh_q4_mm's, bit for bit, for one token, in passes of up to four and
+    in tiles of 16 and 32, whose rows the matrices share."""
     rng = np.random.default_rng(sum(rows) + k)
     ws = [hip.DevBuf(r * (k // 32) * 18) for r in rows]
     for i, (w, r) in enumerate(zip(ws, rows)):
         hip.synth_q4(w, 1, r, k, 7, 50 + i)
-    for n_in in (1, 3):
+    for n_in in (1, 3, 5, 16, 17, 130):
         x = dev((rng.standard_normal((n_in, k)) * 0.5).astype(np.float32))
         ys = [hip.DevBuf(n_in * r * 4) for r in rows]
         hip.q4_mm_n(ws, x, ys, list(rows), k, n_in)
@@ -477,6 +479,8 @@ def test_q4_mm_activation_edge_cases(gpu, n_in):
     (33001, 320, 0),    # 32 rows a wave
     (70001, 256, 0),    # 64 rows a wave for more than 16 tokens, 32 below
     (65537, 96, 0),     # the same, unaligned, in part of one chunk
+    (66001, 2080, 0),   # the same in nine chunks, the last of one block
+    (70001, 2816, 0),   # aligned, in eleven
 ])
 def test_q4_mm_many_rows_token_counts_share_their_bits(gpu, n_out, k, offset):
     """rvh_q4_mm from 16384 rows at the edges of its token tiles: every token of a call has the bits of its
