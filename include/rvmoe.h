@@ -52,9 +52,13 @@ int rvh_event_elapsed(void *start, void *end, float *ms);
 int rvh_rms_norm(const float *x, float *out, const float *weight, int rows, int width, float eps, float post);
 /* y[t][r] = W[r] . x[t], f32 router GEMV; rvhip.h:49-50. */
 int rvh_f32_mm(const float *w, const float *x, float *y, int n_out, int k, int n_in);
-/* y[t][r] = W_q4[r] . x[t], Q4_0 rows (reference layout), f32 activations; rvhip.h:44-45. */
+/* y[t][r] = W_q4[r] . x[t], Q4_0 rows (reference layout), f32 activations; rvhip.h:44-45. The products are
+ * summed in f32 over activations that keep, under 16384 rows, 2^-23 of an element or of the largest of its block of
+ * 32 (two f16; a block 2^60 and more under an earlier one of its row less), and from there (k <= 8192) 2^-28 of that
+ * largest (int8 digits). A token's bits do not depend on the other tokens of the call. A non-finite activation
+ * makes its token's row NaN. */
 int rvh_q4_mm(const void *w, const float *x, float *y, int n_out, int k, int n_in);
-/* rvh_q4_mm's result up to summation order; x 16-byte aligned, w 2-byte aligned; rvhip.h:46-48. */
+/* rvh_q4_mm itself; x 16-byte aligned, w 2-byte aligned; rvhip.h:46-48. */
 int rvh_q4_mv(const void *w, const float *x, float *y, int n_out, int k, int n_in);
 /* n_mat (1 to 4) rvh_q4_mm products on one input in one launch (matrices of 16384 rows or more,
  * k <= 8192, take a launch each): y[m] = w[m] x for matrices of n_out[m] rows (each 2-byte
@@ -77,11 +81,15 @@ int rvh_kv_store(const float *k, const float *v, void *kc, void *vc, int n_tok, 
  * is global, else keys p > pos - window; kv head of query head h is h / (n_head / n_kv).
  * hd % 32 == 0, hd <= 512; the longest key range must be <= max_keys and <= cap. scores is the
  * reference's n_tok * n_head * max_keys scratch: it must be non-NULL and is left untouched (the
- * kernel is rvh_attn_split's with one chunk). rvhip.h:57-60. */
+ * kernels are rvh_attn_split's with one chunk). Scores and sums are f32. A single token's, and few tokens', q and
+ * weighted value scales enter exactly; many tokens share a kernel in which they are two f16 each: q to 2^-23 of an
+ * element or 2^-27 of the largest of its block of 32, a weight times a value scale to 2^-23 of itself or 2^-21 of
+ * the row's largest in that block of the head dimension. There a token's last bits can depend on the other tokens of
+ * the call. rvhip.h:57-60. */
 int rvh_attention(const float *q, const void *kc, const void *vc, float *out, float *scores, int n_tok, int n_head,
                   int n_kv, int hd, int p0, int cap, int window, int max_keys);
-/* Split-K attention, rvh_attention's result up to summation order. Each query's keys are cut into
- * n_chunks contiguous chunks of ceil(keys / n_chunks); n_chunks == 1 writes out (part may be
+/* Split-K attention, rvh_attention's result up to the order and the rounding above. Each query's keys are cut
+ * into n_chunks contiguous chunks of ceil(keys / n_chunks); n_chunks == 1 writes out (part may be
  * NULL), else part receives [n_tok * n_head][n_chunks][hd + 2] = {max, sum, acc[hd]} for
  * rvh_attn_combine. n_chunks <= 65535. rvhip.h:61-65. */
 int rvh_attn_split(const float *q, const void *kc, const void *vc, float *out, float *part, int n_tok, int n_head,

@@ -806,17 +806,17 @@ __global__ __launch_bounds__(ST_WAVES * 64) void k_attn_stream(
 // order (its quants are read transposed, each lane group from its own keys).
 //  - int8 quants are exact in f16;
 //  - q times a power of two of its row (the row's largest lies in [2^14, 2^15)) is the sum of two
-//    f16: 2^-24 of the element, or 2^-40 of the row's largest for smaller ones;
+//    f16: 2^-23 of the element, or 2^-39 of the row's largest for smaller ones;
 //  - p 2^10 likewise, once per stage (p down to 2^-24 has 11 bits or more); a block's p d_v is then
 //    formed in f16 pairs, hi = ph d_v rounded and lo = pl d_v + (ph d_v - hi), whose bracket is exact (a
 //    product of two 11-bit numbers). d_v enters as d_v 2^-E, E the exponent of the largest scale of the
-//    stages so far: exact down to 2^-14 of 2^E, and p d_v to 2^-35 of 2^E.
+//    stages so far: exact down to 2^-14 of 2^E, and p d_v to 2^-33 of 2^E.
 // The last is too little for a row whose own scales lie far below 2^E (another block's, a key's that weighs
-// nothing in it or that it does not see), as 2^-40 of a row's q is for a block of it that meets large key scales.
+// nothing in it or that it does not see), as 2^-39 of a row's q is for a block of it that meets large key scales.
 // So a wave keeps the smallest scale too, and where one of a workgroup's waves met a 0 or a scale under
 // 2^(E - PF_NEAR), or a block of q under 2^-PF_Q of its row, the workgroup walks its stages again: such a
-// block of q has a power of two of its own (2^-28 of the block's largest throughout), and p d_v is formed in f32
-// and scaled by its own power of two per row, block and stage: f16 pairs of 2^-24 of a product, or 2^-40 of
+// block of q has a power of two of its own (2^-27 of the block's largest throughout), and p d_v is formed in f32
+// and scaled by its own power of two per row, block and stage: f16 pairs of 2^-23 of a product, or 2^-39 of
 // the row's largest in the stage. (Both walks, 512 tokens in a window of 1024 keys: 101 us, 53 for one in the
 // same run; 500 tokens x 16 heads of 512 on 4,100 keys 583, 247 for one. The pairs of the second walk in every
 // stage of a single one would cost that much always, and a branch per stage 2 to 5% of the first.)
@@ -826,8 +826,8 @@ __global__ __launch_bounds__(ST_WAVES * 64) void k_attn_stream(
 // round of stages 3.9 us (500 tokens x 16 heads of 512 on 3,601 to 4,100 keys, 247 us, 257 TFLOP/s of
 // the two products; per-token kernel 1244 us); without the copies 3.4 us.
 constexpr int PF_ROWS = 32, PF_KEYS = 32;
-// With every scale in [2^(E - 11), 2^(E + 1)) a row's block has at least 127 2^(E - 12) from the key of its
-// largest weight (p >= 1/2 there), and the 2^-35 2^E of each other key is 2^-23 of that.
+// With every scale in [2^(E - 11), 2^(E + 1)) the key of a row's largest weight (p >= 1/2) has a p d_v of at least
+// 2^(E - 12), and what the other keys' may miss, 2^-33 2^E, is 2^-21 of that.
 constexpr int PF_NEAR = 11, PF_Q = 12;
 // the binary16 bits of 2^(E - PF_NEAR), E >= -15 (1, the smallest scale, if that is below it)
 __device__ __forceinline__ uint32_t pf_near_bits(int E) {

@@ -3,13 +3,13 @@
 // runtime/src/ops.rs:83-92) times f32 activations. The reference's CPU ops are the tolerance target
 // (runtime/tests/hip_ops.rs:56-81).
 //
-// Arithmetic under 16,384 rows, the same for every kernel (from there: k_q4_mm_i8, below), so that a token's result depends neither on the other
-// tokens of the call nor on the launch shape (hip_ops.rs:73-78):
+// Arithmetic under 16,384 rows, the same for every kernel (from there: k_q4_mm_i8, below), so that a token's
+// result depends neither on the other tokens of the call nor on the launch shape (hip_ops.rs:73-78):
 //  - a row's nb blocks fall into four parts of q4_part(nb) blocks;
 //  - the token's activations of a block are scaled by 2^(141 - E), E the largest biased exponent of the
 //    part's blocks up to this one (so that the largest lies under 2^15), or the block's own where that is
-//    more than Q4_NEAR lower (q4_exponent), and split into two f16, each rounded: 2^-24 of the element, or
-//    2^-24 of the block's largest for smaller ones;
+//    more than Q4_NEAR lower (q4_exponent), and split into two f16, each rounded: 2^-23 of the element or
+//    of the block's largest;
 //  - n - 8 is exact in f16, so v_mfma_f32_16x16x32_f16 sums exact products over one block: the low
 //    halves first, the high halves onto them;
 //  - acc = fma(d, sum, acc) in block order from 0; where E changes, acc is first scaled to the new one;
@@ -725,7 +725,7 @@ __global__ __launch_bounds__(QI_WAVES * 64) void k_q4_mm_i8(const uint8_t *__res
 // so with the same bits. Workgroups of 8 waves take 128 RT rows and share the digits of 8 blocks at a
 // time in LDS, formed by the whole workgroup between the 8 before and these. What bounds it: VALU, 7
 // instructions to fold a block's sums per row and token (64 rows and 32 tokens a wave: 262,144 x 2816 in
-// 254 us, 1.7 TB/s of the matrix, 186 TFLOP/s; the folds alone are 137 us of VALU; digits that 16 lanes
+// 254 us, 1.63 TB/s of the matrix, 186 TFLOP/s; the folds alone are 137 us of VALU; digits that 16 lanes
 // read from 512 bytes instead of 128 took 258, 20,000 x 2816 66 instead of 51).
 constexpr int QH_CB = 8;  // blocks per chunk
 template <int NQ, int RT, bool ALN>
