@@ -83,7 +83,7 @@ int rvh_kv_store(const float *k, const float *v, void *kc, void *vc, int n_tok, 
  * reference's n_tok * n_head * max_keys scratch: it must be non-NULL and is left untouched (the
  * kernels are rvh_attn_split's with one chunk). Scores and sums are f32. A single token's, and few tokens', q and
  * weighted value scales enter exactly; many tokens share a kernel in which they are two f16 each: q to 2^-23 of an
- * element or 2^-27 of the largest of its block of 32, a weight times a value scale to 2^-23 of itself or 2^-21 of
+ * element or of the largest of its block of 32, a weight times a value scale to 2^-23 of itself or 2^-21 of
  * the row's largest in that block of the head dimension. There a token's last bits can depend on the other tokens of
  * the call. rvhip.h:57-60. */
 int rvh_attention(const float *q, const void *kc, const void *vc, float *out, float *scores, int n_tok, int n_head,

@@ -815,7 +815,7 @@ __global__ __launch_bounds__(ST_WAVES * 64) void k_attn_stream(
 // nothing in it or that it does not see), as 2^-39 of a row's q is for a block of it that meets large key scales.
 // So a wave keeps the smallest scale too, and where one of a workgroup's waves met a 0 or a scale under
 // 2^(E - PF_NEAR), or a block of q under 2^-PF_Q of its row, the workgroup walks its stages again: such a
-// block of q has a power of two of its own (2^-27 of the block's largest throughout), and p d_v is formed in f32
+// block of q has a power of two of its own (2^-23 of the block's largest throughout), and p d_v is formed in f32
 // and scaled by its own power of two per row, block and stage: f16 pairs of 2^-23 of a product, or 2^-39 of
 // the row's largest in the stage. (Both walks, 512 tokens in a window of 1024 keys: 101 us, 53 for one in the
 // same run; 500 tokens x 16 heads of 512 on 4,100 keys 583, 247 for one. The pairs of the second walk in every
@@ -828,7 +828,7 @@ __global__ __launch_bounds__(ST_WAVES * 64) void k_attn_stream(
 constexpr int PF_ROWS = 32, PF_KEYS = 32;
 // With every scale in [2^(E - 11), 2^(E + 1)) the key of a row's largest weight (p >= 1/2) has a p d_v of at least
 // 2^(E - 12), and what the other keys' may miss, 2^-33 2^E, is 2^-21 of that.
-constexpr int PF_NEAR = 11, PF_Q = 12;
+constexpr int PF_NEAR = 11, PF_Q = 16;
 // the binary16 bits of 2^(E - PF_NEAR), E >= -15 (1, the smallest scale, if that is below it)
 __device__ __forceinline__ uint32_t pf_near_bits(int E) {
     const int e = E - PF_NEAR;
